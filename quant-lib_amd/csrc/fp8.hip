@@ -24,13 +24,15 @@
 // GEMM (quantlib_src/kernels/fp8_gemm.cu:34-139): C[M,N] = A[M,K] W'[N,K]^T with
 // W' the dequantized weights in binary16 and fp32 accumulation.  For few rows the
 // weights are streamed once and dequantized in registers: 1-2 rows as a stream of
-// whole weight rows (v_dot2_f32_f16, no matrix cores), up to 8 rows by whole-row
-// loads into v_mfma_f32_16x16x32_f16, up to 32 rows by the register kernel (each
-// lane 16 codes of a row per chunk), 33-64 rows by whole 128-byte lines re-laid
-// through LDS (C^T = W' A^T, K split over wavefronts and summed in LDS); the
-// in-register dequant multiplies by 1/scale or scales the fp32 sums.  Larger M
+// whole weight rows (v_dot2_f32_f16, no matrix cores), 3-64 rows by whole 128-byte
+// lines re-laid through LDS into v_mfma_f32_16x16x32_f16, K split over wavefronts
+// (stream_gemm.hpp; at 49-64 rows of a large matrix fp8_gemm_wide); K not a
+// multiple of 128, groups not a multiple of 64 and reference-mode E5M2 by the
+// register kernel (each lane 16 codes of a row per chunk).  The in-register
+// dequant multiplies by 1/scale or scales the fp32 sums.  Larger M
 // dequantizes into a workspace with the codec and runs the fp16 library GEMM.
 #include "ql_common.hpp"
+#include "stream_gemm.hpp"
 #include <type_traits>
 #include "quantlib_amd.h"
 
@@ -743,7 +745,7 @@ struct SkinnyArgs {
     _Float16* C;
     float* part;          // [splits][M][N] fp32 partials (splits > 1)
     int M, N, K;
-    int chunks_per_split; // in the kernel's chunks (64 codes; 128 wide, 256 whole-row)
+    int chunks_per_split; // in the kernel's chunks (64 codes; 128 wide)
     long long gs;         // group length in elements
     int groups_per_row;   // K / gs (kScaleGroup)
     int g_step, r_step;   // 256 / gs, 256 % gs: a wavefront's next chunk starts 256 k on
@@ -1340,192 +1342,23 @@ __global__ __launch_bounds__(kBlock) void splitk_reduce(const float* __restrict_
     store<true>(reinterpret_cast<Vec<_Float16, 4>*>(C + i), o);
 }
 
-// ---- one token tile (M <= 16): whole-row weight loads -----------------------------------
-// Workgroup = RW x KW wavefronts over 16*RW weight rows and one K-split: wavefront
-// w owns row tile w % RW and every KW-th chunk of 256 codes from w / RW on.  One
-// load instruction covers 4 complete 256-byte row segments (16 lanes per row): that
-// shape streams the matrix markedly faster than 16 rows x 64 bytes.  Each chunk is
-// re-laid through a wavefront-private LDS tile (16-byte slots XOR-swizzled by row,
-// conflict-free both ways; LDS operations of one wavefront complete in order, so
-// no barrier) into MFMA fragments: lane (row l%16, q = l/16) takes piece p = 0..3
-// from slot 4p + q, i.e. codes 64p + 16q .. +15 of the chunk, and the token
-// fragments use the same k order, so MFMA pair p covers k = 64p .. 64p + 63 of the
-// chunk -- inside one scale group when the group length is a multiple of 64.
-// Token rows come through a buffer resource that ends at row M: lanes of tokens
-// past M read zeros without touching memory.  Scales: per tensor / per row applied
-// once to the sums; per group (length a multiple of 64, dividing K) one multiply-add
-// per output per piece with the inverse from the workgroup's LDS table.  The KW
-// partial tiles of a row tile are summed in LDS in wavefront order.
-constexpr int kRowsChunk = 256;
-constexpr int kRowsStages = 2;        // register ring depth (chunks in flight)
-constexpr int kRowsMaxTokens = 8;     // more tokens: the register path is faster
-constexpr int kRowsOcpWaves = 1024;   // wavefront budgets of the launch shape
-constexpr int kRowsRefWaves = 2048;
-constexpr int kRowsTableFloats = 4096;
-constexpr uint32_t kBufferWord3 = 0x00020000u;          // raw buffer, 32-bit dwords (gfx9)
-
-struct RowsStage {
-    u32x4 w[4];        // instruction i: row 4i + lane/16, bytes 16*(lane%16) .. of the chunk
-    half8 a[4][2];     // piece p: token k = 64p + 16q .. +7 and +8 .. +15 of the chunk
+// ---- 3 to 64 tokens: the weight stream of stream_gemm.hpp -------------------------------
+// One fragment pair of a lane is 16 codes of its row (slot 4h + q of the 128-code
+// chunk), so fragment 2h + e holds codes 64h + 16q + 8e .. +7; the token fragments
+// follow the same order.  Decoded codes only: scales are applied to the sums, which
+// leaves out reference-mode E5M2 (its exponent-31 codes exceed the binary16 range).
+template <int FMT, int MODE>
+struct StreamFp8 {
+    static constexpr int kBytes = 1, kLoads = 2;
+    static __device__ __forceinline__ constexpr int tok_slot(int l, int q) { return 8 * (l >> 1) + 2 * q + (l & 1); }
+    // distinct over any 8 consecutive rows and over the even and the odd rows of 16
+    static __device__ __forceinline__ int swizzle(int row, int col) { return col ^ ((row ^ (row >> 3)) & 7); }
+    static __device__ __forceinline__ void decode(const u32x4 (&v)[2], half8 (&b)[4]) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            dequant16<FMT, MODE, false>(uint4{v[h][0], v[h][1], v[h][2], v[h][3]}, 1.0f, b[2 * h], b[2 * h + 1]);
+    }
 };
-
-__device__ __forceinline__ void rows_load_w(RowsStage& st, const SkinnyArgs& p, const uint32_t (&woff)[4], int c) {
-    const uint32_t kb = (uint32_t)c * kRowsChunk;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) st.w[i] = *reinterpret_cast<const u32x4*>(p.W + (woff[i] + kb));
-}
-
-__device__ __forceinline__ void rows_load_a(RowsStage& st, __amdgpu_buffer_rsrc_t ra, uint32_t aoff, int c) {
-    const uint32_t kb = 2u * (uint32_t)c * kRowsChunk;
-#pragma unroll
-    for (int pc = 0; pc < 4; ++pc) {
-        const u32x4 lo = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + kb + 128u * pc, 0, 0);
-        const u32x4 hi = __builtin_amdgcn_raw_buffer_load_b128(ra, aoff + kb + 128u * pc + 16u, 0, 0);
-        st.a[pc][0] = __builtin_bit_cast(half8, lo);
-        st.a[pc][1] = __builtin_bit_cast(half8, hi);
-    }
-}
-
-template <int FMT, int MODE, int SK, int RW, int KW>
-__global__ __launch_bounds__(RW * KW * kWave) void fp8_gemm_rows(SkinnyArgs p) {
-    constexpr int NW = RW * KW, NR = 16 * RW;
-    // the wavefront index in a scalar register: the chunk loop's branches are uniform
-    const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-    const int rt = wave % RW, kp = wave / RW;
-    const int q = lane >> 4, r16 = lane & 15;
-    const int n0 = blockIdx.x * NR;
-    const int rbase = n0 + 16 * rt;
-    const int n_chunks = p.K / kRowsChunk;
-    const int c_begin = blockIdx.y * p.chunks_per_split;
-    const int c_end = min(n_chunks, c_begin + p.chunks_per_split);
-    uint32_t woff[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) woff[i] = (uint32_t)(rbase + 4 * i + q) * (uint32_t)p.K + 16u * r16;
-    // byte offsets into the token rows; rows past M start at the resource's end
-    // (the host checks (M + 1) * K * 2 < 2^32)
-    const uint32_t a_bytes = 2u * (uint32_t)p.M * (uint32_t)p.K;
-    const uint32_t aoff = (r16 < p.M ? 2u * (uint32_t)r16 * (uint32_t)p.K : a_bytes) + 32u * q;
-    const __amdgpu_buffer_rsrc_t ra =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(p.A), (short)0, (int)a_bytes, (int)kBufferWord3);
-
-    __shared__ u32x4 tile[NW][16][16];
-    __shared__ float table[SK == kScaleGroupFold ? kRowsTableFloats : 1];   // [group - g0][NR rows]
-    __shared__ floatx4 red[KW > 1 ? NW : 1][kWave];
-    int g0 = 0;
-    if constexpr (SK == kScaleGroupFold) {
-        const int gs = (int)p.gs;
-        g0 = c_begin * kRowsChunk / gs;
-        const int ng = (c_end * kRowsChunk - 1) / gs + 1 - g0;   // the host checks NR * ng fits
-        for (int i = threadIdx.x; i < NR * ng; i += NW * kWave) {
-            const int gg = i / NR, rr = i - NR * gg;
-            table[i] = 1.0f / p.scales[(n0 + rr) * p.groups_per_row + g0 + gg];
-        }
-        __syncthreads();
-    }
-
-    floatx4 acc = floatx4{};
-    // one chunk from stage st: re-lay, decode, multiply; with LOAD, the stage is
-    // refilled with chunk c_next (weights as soon as they are in LDS, tokens after
-    // the products)
-    auto step = [&](RowsStage& st, int c, int c_next, auto load) {
-        // re-lay the chunk: row 4i + q, slot r16 -> position r16 ^ row
-#pragma unroll
-        for (int i = 0; i < 4; ++i) tile[wave][4 * i + q][r16 ^ (4 * i + q)] = st.w[i];
-        if constexpr (decltype(load)::value) rows_load_w(st, p, woff, c_next);
-        // orders the compiler only: one wavefront's LDS operations execute in order
-        __builtin_amdgcn_wave_barrier();
-        const u32x4 codes4[4] = {tile[wave][r16][q ^ r16], tile[wave][r16][(4 + q) ^ r16],
-                                 tile[wave][r16][(8 + q) ^ r16], tile[wave][r16][(12 + q) ^ r16]};
-        __builtin_amdgcn_wave_barrier();
-        // pieces of one scale group (groups of 64 codes: every piece; 128: pairs;
-        // 256 and longer: the whole chunk) share one partial and one multiply-add
-        const int gp = SK == kScaleGroupFold ? min(4, (int)p.gs / 64) : 4;   // 1, 2 or 4 (gs % 64 == 0)
-        floatx4 part = floatx4{};
-#pragma unroll
-        for (int pc = 0; pc < 4; ++pc) {
-            const u32x4 cv = codes4[pc];
-            half8 wlo, whi;
-            dequant16<FMT, MODE, false>(uint4{cv[0], cv[1], cv[2], cv[3]}, 1.0f, wlo, whi);
-            if constexpr (SK == kScaleGroupFold) {
-                part = __builtin_amdgcn_mfma_f32_16x16x32_f16(wlo, st.a[pc][0], part, 0, 0, 0);
-                part = __builtin_amdgcn_mfma_f32_16x16x32_f16(whi, st.a[pc][1], part, 0, 0, 0);
-                if ((pc + 1) % gp == 0) {   // wave-uniform
-                    const int g = (c * kRowsChunk + 64 * pc) / (int)p.gs - g0;
-                    const float4 inv = *reinterpret_cast<const float4*>(table + g * NR + 16 * rt + 4 * q);
-                    acc[0] = fmaf(part[0], inv.x, acc[0]);
-                    acc[1] = fmaf(part[1], inv.y, acc[1]);
-                    acc[2] = fmaf(part[2], inv.z, acc[2]);
-                    acc[3] = fmaf(part[3], inv.w, acc[3]);
-                    part = floatx4{};
-                }
-            } else {
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(wlo, st.a[pc][0], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(whi, st.a[pc][1], acc, 0, 0, 0);
-            }
-        }
-        if constexpr (decltype(load)::value) rows_load_a(st, ra, aoff, c_next);
-    };
-    // ring of NS stages: stage s holds the wavefront's chunks s, s + NS, ...  Whole
-    // rounds refill every stage (loads past the last chunk repeat it: in bounds,
-    // never used, and the waits count every round's loads exactly); the remaining
-    // chunks are computed without refills.
-    constexpr int NS = kRowsStages;
-    // wavefront kp of a row tile takes the kp-th contiguous run of the split's chunks
-    constexpr int CS = 1;
-    const int per_w = (c_end - c_begin + KW - 1) / KW;
-    const int first = c_begin + kp * per_w;   // wave-uniform
-    const int w_end = min(c_end, first + per_w);
-    if (first < w_end) {
-        const int n_mine = (w_end - 1 - first) / CS + 1;
-        const int last = first + CS * (n_mine - 1);
-        RowsStage st[NS];
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            rows_load_w(st[s], p, woff, min(first + CS * s, last));
-            rows_load_a(st[s], ra, aoff, min(first + CS * s, last));
-        }
-        const int rounds = n_mine / NS;
-        int c = first;
-        for (int r = 0; r < rounds; ++r) {
-#pragma unroll
-            for (int s = 0; s < NS; ++s, c += CS) step(st[s], c, min(c + CS * NS, last), std::true_type{});
-        }
-#pragma unroll
-        for (int s = 0; s < NS - 1; ++s, c += CS)
-            if (s < n_mine - rounds * NS) step(st[s], c, 0, std::false_type{});
-    }
-    // lane holds C^T[rbase + 4q + i][token r16]; the KW wavefronts of a row tile
-    // are summed in order by the first
-    if constexpr (KW > 1) {
-        red[wave][lane] = acc;
-        __syncthreads();
-        if (kp != 0) return;
-#pragma unroll
-        for (int j = 1; j < KW; ++j) {
-            const floatx4 o = red[rt + RW * j][lane];
-            acc[0] += o[0];
-            acc[1] += o[1];
-            acc[2] += o[2];
-            acc[3] += o[3];
-        }
-    }
-    if constexpr (SK == kScaleTensor || SK == kScaleRow) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[i] *= 1.0f / scale_at<SK>(p, rbase + 4 * q + i, 0);
-    }
-    if (r16 < p.M) {
-        const size_t o = (size_t)r16 * p.N + rbase + 4 * q;
-        if (gridDim.y == 1) {
-            Vec<_Float16, 4> h;
-#pragma unroll
-            for (int i = 0; i < 4; ++i) h.v[i] = from_f32<_Float16>(acc[i]);
-            *reinterpret_cast<Vec<_Float16, 4>*>(p.C + o) = h;
-        } else {
-            *reinterpret_cast<float4*>(p.part + (size_t)blockIdx.y * p.M * p.N + o) =
-                float4{acc[0], acc[1], acc[2], acc[3]};
-        }
-    }
-}
 
 // ---- one or two tokens: contiguous row streams -----------------------------------------
 // At most kVecMaxTokens tokens the GEMM is a stream of the weight matrix, and the
@@ -1770,7 +1603,6 @@ inline size_t align256(size_t n) { return (n + 255) & ~size_t(255); }
 
 struct SkinnyPlan {
     int mt, r, splits, chunks_per_split;
-    int rw = 0, kw = 0;   // whole-row path: row tiles per workgroup, wavefronts per row tile
 };
 
 SkinnyPlan skinny_plan(int M, int N, int K, size_t ws_bytes) {
@@ -1908,77 +1740,114 @@ void launch_gemv(const SkinnyArgs& a, int kind, int J, hipStream_t st) {
         launch_gemv_sk<FMT, MODE, kScaleGroupFold>(a, J, st);
 }
 
-// Whole-row path for one token tile: chunks of 256 codes, scales per tensor, per
-// row or per group of a multiple of 64 codes dividing K (the group table of a split
-// must fit LDS).  It multiplies decoded codes and scales the sums, so
-// reference-mode E5M2 (whose exponent-31 codes decode beyond the binary16 range)
-// stays on the register path.
-int rows_kind(const Geom& g, int M, int N, int K, int format, int mode) {
-    if (M > kRowsMaxTokens || N % 16 || K % kRowsChunk || (format == QL_FP8_E5M2 && mode == QL_FP8_MODE_REFERENCE) ||
-        (uint64_t)(M + 1) * (uint64_t)K * 2u >= (1ull << 32))
+// Launch shape of the stream kernel: 16 * r weight rows and nw wavefronts per
+// workgroup, K over `splits` workgroups (r = 0: the kernel does not apply).
+struct StreamPlan {
+    int r = 0, nw = 8, splits = 1, chunks_per_split = 0;
+};
+
+// The kernel's scale kind (kStreamRow also covers per tensor), or -1.
+int stream_kind(const Geom& g, int M, int N, int K, int format, int mode) {
+    if (M > 64 || N % 16 || K % kStreamChunk || K > kStreamMaxK || (format == QL_FP8_E5M2 && mode == QL_FP8_MODE_REFERENCE))
         return -1;
-    if (g.n_groups == 1) return kScaleTensor;
-    if (g.gs == K) return kScaleRow;
+    if (g.n_groups == 1 || g.gs == K) return kStreamRow;
     if (K % g.gs || g.gs % 64) return -1;
-    return kScaleGroupFold;
+    return g.gs % kStreamChunk ? kStreamHalfGroup : kStreamGroup;
 }
 
-// Shape of the whole-row launch: KW (wavefronts sharing a row tile, splitting its
-// chunks) is the largest of 1, 2, 4, 8 that keeps N/16 * KW wavefronts within
-// max_waves and gives every wavefront at least a ring of chunks; RW = 4 / KW row
-// tiles per workgroup (1 for KW >= 4), lowered until N divides.  K-splits over
-// launches (fp32 partials + splitk_reduce) only when KW = 8 leaves the chip
-// short of wavefronts.  Measured on MI355X with weights streamed from HBM:
-// about 1024 wavefronts suit the OCP decode, about 2048 the reference-mode decode
-// (its check of every code needs more wavefronts to hide).
-SkinnyPlan rows_plan(int M, int N, int K, int mode, size_t ws_bytes) {
-    const int max_waves = mode == QL_FP8_MODE_REFERENCE ? kRowsRefWaves : kRowsOcpWaves;
-    SkinnyPlan s;
-    const int tiles = N / 16;
-    const int n_chunks = K / kRowsChunk;
-    s.kw = 1;
-    while (s.kw < 8 && tiles * 2 * s.kw <= max_waves && n_chunks / (2 * s.kw) >= kRowsStages) s.kw *= 2;
-    s.rw = s.kw >= 4 ? 1 : 4 / s.kw;
-    while (tiles % s.rw) s.rw /= 2;
-    s.mt = 1;
-    s.r = s.rw;
+// Every workgroup reads all token rows of its K range, so the rows per workgroup and
+// the K-split trade the number of workgroups against that traffic.  Measured on
+// MI355X, weights streamed from HBM, E4M3 groups of 128 checked clean (us per call,
+// r x splits x nw; last: the kernel that ran there before):
+//   4096 x 4096, 8 / 32 tokens   1x1x8  7.2 / 10.0   2x2x8  8.0 / 10.7   (7.4 / 13.3)
+//   4096 x 14336, 4 / 16 / 32    1x1x8 14.6 / 17.5 / 25.9   4x4x4 15.9 / 17.5 / 20.7   (15.6 / 21.8 / 26.2)
+//   2048 x 14336, 4 / 32 / 48    1x1x8 13.8 / 24.7 / 31.5   1x4x4 11.7 / 17.5 / 21.0   (14.0 / 19.0 / 20.0)
+//   1024 x 4096, 4 / 32          1x1x8  5.9 /  9.1   1x4x4  6.4 /  7.4   (6.3 / 13.1)
+//   6144 x 4096, 8 / 32 / 64     2x1x8  8.4 / 12.7 / 16.9   4x1x4 12.9 / 17.1 / 23.5   (10.3 / 16.5 / 18.5)
+//   8192 x 8192, 16 / 32 / 48    2x1x8 20.2 / 22.8 / 26.5   4x1x4 25.3 / 30.8 / 35.6   (22.9 / 26.6 / 28.0)
+//   14336 x 4096, 4 / 16 / 32 / 48   4x1x4 14.5 / 16.1 / 19.3 / 23.2   2x1x8 15.8 / 17.3 / 23.4 / 28.1
+//                                    (16.4 / 19.3 / 23.3 / 23.8)
+// With four token tiles the whole-line kernel is faster from 10000 rows on (25.1
+// against 26.7 us at 14336 x 4096) and where the tokens are large (26.6 against 27.2
+// at 4096 x 14336).
+constexpr int kStreamWideN = 10000;
+constexpr int kStreamTokBytes = 300 * 1024;   // tokens that every workgroup may re-read
+
+StreamPlan stream_plan(int M, int N, int K, size_t ws_bytes) {
+    StreamPlan s;
+    const int n_chunks = K / kStreamChunk;
+    const bool large = (long long)M * K * 2 > kStreamTokBytes;
+    if (M > 48 && (N >= kStreamWideN || (N <= 4096 && (long long)M * K * 2 > 2 * kStreamTokBytes))) return s;
+    s.r = 1;
     int splits = 1;
-    if (s.kw == 8 && tiles * 16 <= max_waves)
-        splits = std::min(max_waves / (tiles * 8), std::max(1, n_chunks / (8 * kRowsStages)));
-    while (splits > 1 && (size_t)splits * (size_t)M * (size_t)N * sizeof(float) > ws_bytes) --splits;
+    if (N >= kStreamWideN) {
+        s.r = 4;
+        s.nw = 4;
+    } else if (N > 4096) {
+        s.r = 2;
+    } else if (large && M <= 48) {
+        s.r = N >= 3072 ? 4 : 1;
+        s.nw = N >= 3072 ? 4 : 8;
+        splits = std::min(N >= 3072 ? 256 / ((N + 63) / 64) : 4, std::max(1, n_chunks / (2 * s.nw)));
+        while (splits > 1 && (size_t)splits * (size_t)M * (size_t)N * sizeof(float) > ws_bytes) --splits;
+        if (splits == 1) {
+            s.r = 1;
+            s.nw = 8;
+        }
+    }
     s.chunks_per_split = (n_chunks + splits - 1) / splits;
     s.splits = (n_chunks + s.chunks_per_split - 1) / s.chunks_per_split;
     return s;
 }
 
-// largest number of scale groups one K-split of the plan touches
-int rows_groups_per_split(const SkinnyPlan& pl, int K, long long gs) {
-    const int n_chunks = K / kRowsChunk;
-    int ng_max = 0;
-    for (int s = 0; s < pl.splits; ++s) {
-        const int cb = s * pl.chunks_per_split, ce = std::min(n_chunks, cb + pl.chunks_per_split);
-        ng_max = std::max(ng_max, (int)((ce * (long long)kRowsChunk - 1) / gs + 1 - cb * (long long)kRowsChunk / gs));
+template <int FMT, int MODE, int SK, int MT>
+void launch_stream_mt(const StreamArgs& a, const StreamPlan& pl, hipStream_t st) {
+    using WP = StreamFp8<FMT, MODE>;
+    const dim3 grid(qlh::blocks_for(a.N, 16 * pl.r), (unsigned)pl.splits), block(pl.nw * kWave);
+    if (pl.r == 4) {
+        if constexpr (MT < 4) hipLaunchKernelGGL((stream_gemm<WP, SK, MT, 4, 4>), grid, block, 0, st, a);
+    } else if (pl.r == 2) {
+        hipLaunchKernelGGL((stream_gemm<WP, SK, MT, 2, 8>), grid, block, 0, st, a);
+    } else {
+        hipLaunchKernelGGL((stream_gemm<WP, SK, MT, 1, 8>), grid, block, 0, st, a);
     }
-    return ng_max;
 }
 
-template <int FMT, int MODE, int RW, int KW>
-void launch_rows_shape(const SkinnyArgs& a, const SkinnyPlan& pl, int kind, hipStream_t st) {
-    const dim3 grid((unsigned)(a.N / (16 * RW)), (unsigned)pl.splits), block(RW * KW * kWave);
-    if (kind == kScaleTensor) hipLaunchKernelGGL((fp8_gemm_rows<FMT, MODE, kScaleTensor, RW, KW>), grid, block, 0, st, a);
-    else if (kind == kScaleRow) hipLaunchKernelGGL((fp8_gemm_rows<FMT, MODE, kScaleRow, RW, KW>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((fp8_gemm_rows<FMT, MODE, kScaleGroupFold, RW, KW>), grid, block, 0, st, a);
+template <int FMT, int MODE, int SK>
+void launch_stream_sk(const StreamArgs& a, const StreamPlan& pl, hipStream_t st) {
+    switch ((a.M + 15) / 16) {
+    case 1: launch_stream_mt<FMT, MODE, SK, 1>(a, pl, st); break;
+    case 2: launch_stream_mt<FMT, MODE, SK, 2>(a, pl, st); break;
+    case 3: launch_stream_mt<FMT, MODE, SK, 3>(a, pl, st); break;
+    default: launch_stream_mt<FMT, MODE, SK, 4>(a, pl, st); break;
+    }
 }
 
 template <int FMT, int MODE>
-void launch_rows(const SkinnyArgs& a, const SkinnyPlan& pl, int kind, hipStream_t st) {
-    if (pl.kw == 8) launch_rows_shape<FMT, MODE, 1, 8>(a, pl, kind, st);
-    else if (pl.kw == 4) launch_rows_shape<FMT, MODE, 1, 4>(a, pl, kind, st);
-    else if (pl.kw == 2 && pl.rw == 2) launch_rows_shape<FMT, MODE, 2, 2>(a, pl, kind, st);
-    else if (pl.kw == 2) launch_rows_shape<FMT, MODE, 1, 2>(a, pl, kind, st);
-    else if (pl.rw == 4) launch_rows_shape<FMT, MODE, 4, 1>(a, pl, kind, st);
-    else if (pl.rw == 2) launch_rows_shape<FMT, MODE, 2, 1>(a, pl, kind, st);
-    else launch_rows_shape<FMT, MODE, 1, 1>(a, pl, kind, st);
+void launch_stream(const StreamArgs& a, const StreamPlan& pl, int kind, hipStream_t st) {
+    if constexpr (!(FMT == QL_FP8_E5M2 && MODE == QL_FP8_MODE_REFERENCE)) {   // stream_kind() leaves it out
+        if (kind == kStreamRow) launch_stream_sk<FMT, MODE, kStreamRow>(a, pl, st);
+        else if (kind == kStreamGroup) launch_stream_sk<FMT, MODE, kStreamGroup>(a, pl, st);
+        else launch_stream_sk<FMT, MODE, kStreamHalfGroup>(a, pl, st);
+    }
+}
+
+// Workspace reserved for at most 8 tokens with K a multiple of 256 (K-splits of
+// 16-row tiles over 2048 wavefronts): more than stream_plan() uses there, kept so
+// that ql_fp8_gemm_workspace_size reports the sizes it always has.
+int reserved_splits(const Geom& g, int M, int N, int K) {
+    if (M > 8 || N % 16 || K % 256 || (uint64_t)(M + 1) * (uint64_t)K * 2u >= (1ull << 32)) return 1;
+    if (g.n_groups != 1 && g.gs != K && (K % g.gs || g.gs % 64)) return 1;
+    int most = 1;
+    for (int waves : {1024, 2048}) {
+        const int tiles = N / 16, n = K / 256;
+        int kw = 1;
+        while (kw < 8 && tiles * 2 * kw <= waves && n / (2 * kw) >= 2) kw *= 2;
+        int splits = kw == 8 && tiles * 16 <= waves ? std::min(waves / (tiles * 8), std::max(1, n / 16)) : 1;
+        const int per = (n + splits - 1) / splits;
+        most = std::max(most, (n + per - 1) / per);
+    }
+    return most;
 }
 
 // the register path addresses W and A with 32-bit byte offsets
@@ -2175,13 +2044,8 @@ extern "C" hipError_t ql_fp8_gemm_workspace_size(int M, int N, int K, int granul
     *bytes = 0;
     if (M == 0 || N == 0 || K == 0) return hipSuccess;
     if (skinny_ok(M, N, K, g)) {
-        // the format and mode only narrow the whole-row path's group case; the
-        // reservation covers either path
         const SkinnyPlan pl = skinny_plan(M, N, K, SIZE_MAX);
-        size_t splits = (size_t)pl.splits;
-        if (rows_kind(g, M, N, K, QL_FP8_E4M3, QL_FP8_MODE_OCP) >= 0)
-            for (int mode : {QL_FP8_MODE_REFERENCE, QL_FP8_MODE_OCP})
-                splits = std::max(splits, (size_t)rows_plan(M, N, K, mode, SIZE_MAX).splits);
+        const size_t splits = (size_t)std::max(pl.splits, reserved_splits(g, M, N, K));
         *bytes = splits > 1 ? splits * (size_t)M * (size_t)N * sizeof(float) : 0;
         if (pl.mt == 4) *bytes = align256(*bytes) + packed_a_bytes(K, pl.mt);   // fragment-major tokens
     } else {
@@ -2219,12 +2083,28 @@ extern "C" hipError_t ql_fp8_gemm_f16(const uint16_t* A, const uint8_t* W, const
     if (skinny_ok(M, N, K, g) && qlh::aligned16(A) && qlh::aligned16(W)) {
         const bool ws_ok = workspace && qlh::aligned16(workspace) && ((uintptr_t)C & 7) == 0;
         const size_t ws = ws_ok ? workspace_bytes : 0;
-        int rkind = rows_kind(g, M, N, K, format, mode);
-        SkinnyPlan pl = rkind >= 0 ? rows_plan(M, N, K, mode, ws) : skinny_plan(M, N, K, ws);
-        if (rkind == kScaleGroupFold && 16LL * pl.rw * rows_groups_per_split(pl, K, g.gs) > kRowsTableFloats) {
-            rkind = -1;
-            pl = skinny_plan(M, N, K, ws);
+        const int skind = stream_kind(g, M, N, K, format, mode);
+        const StreamPlan sp = skind >= 0 ? stream_plan(M, N, K, ws) : StreamPlan{};
+        if (sp.r > 0) {
+            StreamArgs a{};
+            a.A = reinterpret_cast<const char*>(A);
+            a.W = reinterpret_cast<const char*>(W);
+            a.scales = scales;
+            a.C = reinterpret_cast<_Float16*>(C);
+            a.M = M;
+            a.N = N;
+            a.K = K;
+            a.gs = (int)std::min<long long>(g.gs, K);
+            a.groups_per_row = g.n_groups == 1 ? 0 : K / a.gs;
+            a.part = static_cast<float*>(workspace);
+            a.chunks_per_split = sp.chunks_per_split;
+            QL_FP8_DISPATCH(format, mode, launch_stream, a, sp, skind, stream);
+            if (sp.splits > 1)
+                hipLaunchKernelGGL(splitk_reduce, dim3(qlh::blocks_for((long long)M * N / 4, kBlock)), dim3(kBlock), 0,
+                                   stream, a.part, a.C, sp.splits, (long long)M * N);
+            return hipGetLastError();
         }
+        SkinnyPlan pl = skinny_plan(M, N, K, ws);
         // more than 32 tokens (four token tiles) on the register path: the token
         // rows are copied fragment-major after the split partials, when the
         // workspace holds both, and the whole-line kernel reads them where it
@@ -2236,18 +2116,16 @@ extern "C" hipError_t ql_fp8_gemm_f16(const uint16_t* A, const uint8_t* W, const
         // 24.9 / 28.5 (the fp16 library GEMM: 26.5 / 29.7).  At 32 rows the
         // copy's launch cost more than it saved (+3-4%).
         const size_t part_bytes = pl.splits > 1 ? (size_t)pl.splits * (size_t)M * (size_t)N * sizeof(float) : 0;
-        const bool pack_fits = rkind < 0 && pl.mt == 4 && ws_ok &&
+        const bool pack_fits = pl.mt == 4 && ws_ok &&
                                align256(part_bytes) + packed_a_bytes(K, pl.mt) <= workspace_bytes;
         // the whole-line kernel where it applies, reading the token rows itself or
         // (wide_token_stages 0) the copy; else the register kernel, on the copy when
         // the workspace holds it
-        int kind = -1, wk = -1, cps = 0, wsplits = 0;
-        if (rkind < 0) {
-            kind = scale_kind(g, K, pl, format, mode);
-            const bool fold_ok = !(format == QL_FP8_E5M2 && mode == QL_FP8_MODE_REFERENCE);
-            wk = wide_kind(g, K, pl, kind, fold_ok, cps, wsplits);
-            if (wk >= 0 && wide_token_stages(mode, wk) == 0 && !pack_fits) wk = -1;
-        }
+        int cps = 0, wsplits = 0;
+        const int kind = scale_kind(g, K, pl, format, mode);
+        const bool fold_ok = !(format == QL_FP8_E5M2 && mode == QL_FP8_MODE_REFERENCE);
+        int wk = wide_kind(g, K, pl, kind, fold_ok, cps, wsplits);
+        if (wk >= 0 && wide_token_stages(mode, wk) == 0 && !pack_fits) wk = -1;
         const bool pack = pack_fits && (wk < 0 || wide_token_stages(mode, wk) == 0);
         SkinnyArgs a;
         a.A = reinterpret_cast<const char*>(A);
@@ -2272,23 +2150,12 @@ extern "C" hipError_t ql_fp8_gemm_f16(const uint16_t* A, const uint8_t* W, const
         a.groups_per_row = K % g.gs == 0 ? (int)(K / g.gs) : 0;
         a.g_step = (int)(256 / g.gs);
         a.r_step = (int)(256 % g.gs);
-        if (rkind >= 0) {
-            // rows_kind() keeps reference-mode E5M2 on the register path
-            if (format == QL_FP8_E4M3 && mode == QL_FP8_MODE_REFERENCE)
-                launch_rows<QL_FP8_E4M3, QL_FP8_MODE_REFERENCE>(a, pl, rkind, stream);
-            else if (format == QL_FP8_E4M3)
-                launch_rows<QL_FP8_E4M3, QL_FP8_MODE_OCP>(a, pl, rkind, stream);
-            else if (mode == QL_FP8_MODE_OCP)
-                launch_rows<QL_FP8_E5M2, QL_FP8_MODE_OCP>(a, pl, rkind, stream);
-            else
-                return hipErrorInvalidValue;
+        if (wk >= 0) {
+            a.chunks_per_split = cps;
+            pl.splits = wsplits;
+            QL_FP8_DISPATCH(format, mode, launch_wide, a, wk, wsplits, stream);
         } else {
-            if (wk >= 0) {
-                a.chunks_per_split = cps;
-                pl.splits = wsplits;
-                QL_FP8_DISPATCH(format, mode, launch_wide, a, wk, wsplits, stream);
-            } else
-                QL_FP8_DISPATCH(format, mode, launch_skinny, a, pl, kind, stream);
+            QL_FP8_DISPATCH(format, mode, launch_skinny, a, pl, kind, stream);
         }
         if (pl.splits > 1) {
             const long long mn = (long long)M * N;

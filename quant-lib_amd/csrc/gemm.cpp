@@ -1,6 +1,7 @@
 // gemm.cpp -- the fp16 library GEMM used by the layer engine and the FP8 GEMM's
 // large-M path: y[M, N] = x[M, K] W[N, K]^T (row-major, weights [out, in]),
-// fp16 in/out, fp32 accumulation, on hipBLASLt.
+// fp16 in/out, fp32 accumulation, on hipBLASLt; at most 16 rows by the weight-stream
+// kernel where it is the faster one (gemm_stream.hip).
 //
 // Column-major view for the library: y^T (N x M) = op(A) op(B) with A = W stored
 // K x N and transposed, B = x stored K x M.  Plans (descriptors + the heuristic's
@@ -10,6 +11,7 @@
 // process ends.  ql_gemm_tune_f16 replaces a shape's algorithm by the fastest of
 // the heuristic's candidates, timed on scratch operands.
 #include "quantlib_amd.h"
+#include "gemm_stream.hpp"
 
 #include <hipblaslt/hipblaslt.h>
 
@@ -92,6 +94,7 @@ extern "C" hipError_t ql_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t
     if (M < 0 || N < 0 || K < 0) return hipErrorInvalidValue;
     if (M == 0 || N == 0) return hipSuccess;
     if (!x || !w || !y || K == 0) return hipErrorInvalidValue;
+    if (qlh::stream_gemm_f16_applies(x, w, M, N, K)) return qlh::stream_gemm_f16(x, w, y, M, N, K, stream);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return hipErrorNoDevice;
     Plan plan;

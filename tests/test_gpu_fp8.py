@@ -529,3 +529,45 @@ def test_gemm_f16_matches_oracle(M, N, K):
     exact = gemm_exact(a, w)
     check_gemm(orc.matmul(a, w), exact, "oracle")
     check_gemm(host(out, shape=(M, N)), exact, f"gemm {M}x{N}x{K}")
+
+
+# The weight-stream GEMM (3 to 64 tokens, K a multiple of 128, scales per tensor, per
+# row or in groups of a multiple of 64): every number of token tiles with full and
+# ragged last tiles, 1, 2 and 4 row tiles per workgroup with a ragged last workgroup
+# (N = 80, 4112, 10064), fewer chunks than wavefronts, and K-splits of unequal length
+# of both split shapes (with the workspace; without one they run unsplit).
+STREAM_GEMM_SHAPES = [
+    (3, 80, 128), (16, 80, 1152), (17, 80, 1280), (48, 48, 384), (64, 80, 2176),
+    (4, 4112, 128), (31, 4112, 256), (33, 4112, 128), (49, 4112, 384),
+    (5, 10064, 128), (32, 10064, 256), (47, 10064, 384),
+    (33, 3088, 4736), (48, 80, 9600), (17, 96, 9088)]
+
+
+@pytest.mark.parametrize("fmt,mode", [(ql.FP8_E4M3, ql.FP8_MODE_REFERENCE), (ql.FP8_E4M3, ql.FP8_MODE_OCP),
+                                      (ql.FP8_E5M2, ql.FP8_MODE_OCP)])
+@pytest.mark.parametrize("gran,gs", [(ql.QUANT_PER_TENSOR, 0), (ql.QUANT_PER_CHANNEL, 0), (ql.QUANT_PER_GROUP, 128),
+                                     (ql.QUANT_PER_GROUP, 64)])
+@pytest.mark.parametrize("M,N,K", STREAM_GEMM_SHAPES)
+def test_fp8_gemm_weight_stream(M, N, K, gran, gs, fmt, mode):
+    a = to_f16_bits(normal(7 * M + N + K, (M, K)))
+    w = to_f16_bits(normal(3 * N + K, (N, K), K ** -0.5))
+    q, sc = orc.fp8_quantize(w, fmt, gran, gs, mode)
+    exact = gemm_exact(a, orc.fp8_dequantize(q, sc, fmt, gran, gs, mode))
+    for workspace in ("query", "none"):
+        got = gpu_fp8_gemm(a, q, sc, M, N, K, fmt, gran, gs, mode, workspace)
+        check_gemm(got, exact, f"fp8 gemm {M}x{N}x{K} gran {gran} gs {gs} workspace {workspace}")
+
+
+# The same kernel on binary16 weights (at most 16 tokens): 1, 2 and 4 row tiles per
+# workgroup with ragged last workgroups and any N, and operands off 16-byte alignment,
+# which the library takes.
+@pytest.mark.parametrize("M,N,K,shift", [(1, 17, 128, 0), (16, 33, 1152, 0), (5, 4097, 256, 0), (15, 4130, 2048, 0),
+                                         (16, 12305, 384, 0), (8, 12305, 128, 0), (9, 13000, 128, 0), (3, 128, 256, 1)])
+def test_gemm_f16_weight_stream(M, N, K, shift):
+    a = to_f16_bits(normal(M + K, (M, K)))
+    w = to_f16_bits(normal(N + K, (N, K), K ** -0.5))
+    da = dev(np.concatenate([np.zeros(shift, np.uint16), a.reshape(-1)]))
+    dw = dev(w)
+    out = empty((M * N,), np.uint16)
+    ql.call("ql_gemm_f16", da.ptr + 2 * shift, dw.ptr, out.ptr, M, N, K, stream())
+    check_gemm(host(out, shape=(M, N)), gemm_exact(a, w), f"gemm {M}x{N}x{K}")
