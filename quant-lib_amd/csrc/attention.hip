@@ -13,9 +13,10 @@
 // reference's tiles hold 64) and any other value up to 64 on a vector-ALU
 // kernel (attn_small), rows may be strided, and K/V may live in 16-token pages.
 //
-// Work decomposition (prefill).  One workgroup = 4 wavefronts = 128
-// consecutive queries of one query head; each wavefront owns 32 queries.  Keys
-// stream through LDS in tiles of 64, loaded straight from global memory into
+// Work decomposition (prefill).  One workgroup = 4 wavefronts that share a KV
+// head; each wavefront owns 32 queries of one query head (the heads of a KV head
+// side by side, prefill_item).  Small launches give a workgroup two such groups,
+// each with half the key tiles (fwd_two_groups).  Keys stream through LDS in tiles of 64, loaded straight from global memory into
 // the other of two LDS stages while the current tile is multiplied.  Per tile
 // and wavefront:
 //   S^T (64 keys x 32 queries) = K . Q^T    -- v_mfma_f32_32x32x16_f16
@@ -63,7 +64,8 @@ typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int kAttnWaves = 4;
 constexpr int kAttnThreads = kAttnWaves * kWave;   // 256
-constexpr int kBQ = 32 * kAttnWaves;               // 128 queries per workgroup
+constexpr int kWaveQ = 32;                         // queries of a prefill wavefront
+constexpr int kOneGroupTiles = 4;                  // key tiles that two wavefront groups do not split
 constexpr int kBK = 64;                            // keys per tile
 
 // Pair reductions across lanes l and l ^ 32 (l ^ 16) without an LDS round
@@ -393,23 +395,36 @@ __device__ __forceinline__ half4 lds_read_tr4(const _Float16* p) {
     return __builtin_bit_cast(half4, r);
 }
 
-// Work item of a prefill workgroup: (query head, query tile).  Consecutive
-// workgroup ids go to the 8 XCDs in turn; when the heads split evenly over the
-// XCDs, each XCD is given its own contiguous run of heads (so the K/V rows of
-// their shared KV heads stay in that XCD's L2).  Causal: heavy (late) query
-// tiles first.
-__device__ __forceinline__ void prefill_item(const AttnArgs& a, int& head, int& qt) {
-    const int n_qt = (int)gridDim.x / a.n_heads;
+// Work items of the prefill.  A slot is 32 queries of one query head, one
+// wavefront's work; the slots of a KV head are numbered query block by query block,
+// the heads that share it in turn, and a workgroup takes four consecutive ones.  So
+// with four heads a KV head its wavefronts hold the same 32 queries and see the same
+// keys: a prompt is padded to 32 rows instead of 128, and no wavefront idles at the
+// causal edge.  (Heads that do not split evenly over the KV heads: one head's slots.)
+__host__ __device__ inline int fwd_heads_per_item(int n_heads, int n_kv_heads) {
+    return n_heads % n_kv_heads == 0 ? n_heads / n_kv_heads : 1;
+}
+
+// KV head (or, ungrouped, query head) and quadruple of slots of a workgroup.
+// Consecutive workgroup ids go to the 8 XCDs in turn; when the heads split evenly
+// over the XCDs, or the XCDs over the heads, each XCD is given its own heads (so
+// their K/V rows stay in that XCD's L2).  Causal: heavy (late) queries first.
+__device__ __forceinline__ void prefill_item(const AttnArgs& a, int n_items, int& item, int& quad) {
+    const int n_quads = (int)gridDim.x / n_items;
+    const int id = (int)blockIdx.x, xcd = id & 7, j = id >> 3;
     int t;
-    if (a.n_heads % 8 == 0) {
-        const int hpx = a.n_heads / 8, xcd = (int)blockIdx.x & 7, j = (int)blockIdx.x >> 3;
-        head = xcd * hpx + j % hpx;
-        t = j / hpx;
+    if (n_items % 8 == 0) {
+        const int ipx = n_items / 8;
+        item = xcd * ipx + j % ipx;
+        t = j / ipx;
+    } else if (8 % n_items == 0 && n_quads % (8 / n_items) == 0) {
+        item = xcd % n_items;
+        t = j * (8 / n_items) + xcd / n_items;
     } else {
-        head = (int)blockIdx.x % a.n_heads;
-        t = (int)blockIdx.x / a.n_heads;
+        item = id % n_items;
+        t = id / n_items;
     }
-    qt = a.causal ? n_qt - 1 - t : t;
+    quad = a.causal ? n_quads - 1 - t : t;
 }
 
 // Q^T operand: lane holds Q[query][d = 16*kk + 8*hh + 0..7] (zeros past the last query).
@@ -516,29 +531,45 @@ __device__ __forceinline__ void store_o(const floatx16 (&o)[HD / 32], float l_ru
     }
 }
 
-// One prefill workgroup: 128 queries of one query head against every key they
-// see, in 64-key tiles through two LDS stages.  The stages are two distinct
+// The sequence of grid plane z, in order of falling key counts (the workgroups of
+// a later plane start later): up to 64 sequences, ranked by every wavefront.
+__device__ __forceinline__ int longest_first(const int32_t* ctx_lens, int n, int z) {
+    if (n > kWave) return z;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int len = ctx_lens[min(lane, n - 1)];
+    int rank = 0;
+    for (int i = 0; i < n; ++i) {
+        const int other = __builtin_amdgcn_readlane(len, i);
+        rank += other > len || (other == len && i < lane);
+    }
+    return __builtin_ctzll(__ballot(lane < n && rank == z));
+}
+
+// One prefill workgroup: four slots of 32 queries against every key they see, in
+// 64-key tiles through two LDS stages.  G = 2: two groups of four
+// wavefronts take alternate tiles, each through stages of its own, and their
+// (maximum, sum, O) are merged through LDS at the end.  The stages are two distinct
 // arrays and the tile loop is unrolled by two, so no wait for the loads into
 // one stage is placed before the reads of the other.  Paged K/V: wavefront w
 // loads page w of each tile, and the base of its page of tile t+2 is looked up
 // (WavePagePipe) while tile t is multiplied.
-template <int HD, bool PAGED, bool NARROW = false>
-__global__ __launch_bounds__(kAttnThreads, 2) void attn_fwd(AttnArgs a) {
+template <int HD, bool PAGED, bool NARROW = false, int G = 1>
+__global__ __launch_bounds__(G * kAttnThreads, 2) void attn_fwd(AttnArgs a) {
     using T = KvTile<HD>;
     constexpr int NKK = HD / 16;   // MFMA steps over d for S^T
     constexpr int NDB = HD / 32;   // 32-row blocks of O^T
-    __shared__ __attribute__((aligned(16))) _Float16 sk0[T::ELEMS];
-    __shared__ __attribute__((aligned(16))) _Float16 sv0[T::ELEMS];
-    __shared__ __attribute__((aligned(16))) _Float16 sk1[T::ELEMS];
-    __shared__ __attribute__((aligned(16))) _Float16 sv1[T::ELEMS];
+    __shared__ __attribute__((aligned(16))) _Float16 sk0[G * T::ELEMS];
+    __shared__ __attribute__((aligned(16))) _Float16 sv0[G * T::ELEMS];
+    __shared__ __attribute__((aligned(16))) _Float16 sk1[G * T::ELEMS];
+    __shared__ __attribute__((aligned(16))) _Float16 sv1[G * T::ELEMS];
 
-    int head, qt;
-    prefill_item(a, head, qt);
-    const int kvh = (int)(((long long)head * a.n_kv_heads) / a.n_heads);
+    const int per_item = fwd_heads_per_item(a.n_heads, a.n_kv_heads);
+    int item, quad;
+    prefill_item(a, a.n_heads / per_item, item, quad);
     int q_begin = 0, q_len = a.q_len, kv_len = a.kv_len;
     const int32_t* table = nullptr;
     if constexpr (PAGED) {
-        const int s = blockIdx.z;
+        const int s = G > 1 && gridDim.z > 1 ? longest_first(a.ctx_lens, (int)gridDim.z, (int)blockIdx.z) : (int)blockIdx.z;
         q_begin = a.cu_q[s];
         q_len = a.cu_q[s + 1] - q_begin;
         kv_len = a.ctx_lens[s];
@@ -546,29 +577,36 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_fwd(AttnArgs a) {
         if (kv_len > a.max_blocks * QL_PAGE_SIZE) kv_len = a.max_blocks * QL_PAGE_SIZE;
         table = a.block_tables + (size_t)s * a.max_blocks;
     }
-    const int q0 = qt * kBQ;
-    if (q0 >= q_len) return;   // workgroup-uniform
+    if (quad * kAttnWaves / per_item * kWaveQ >= q_len) return;   // workgroup-uniform
     if (kv_len < 0) kv_len = 0;
 
     const int lane = threadIdx.x & (kWave - 1);
     // paged: a scalar wave index makes load_tile's page choice scalar (the
     // compiler's register allocation measured best this way for each layout)
-    const int wave = PAGED ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave) : (int)threadIdx.x / kWave;
+    const int wave_id = PAGED || G > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave) : (int)threadIdx.x / kWave;
+    const int wave = G > 1 ? wave_id % kAttnWaves : wave_id;   // within its group
+    const int grp_id = G > 1 ? wave_id / kAttnWaves : 0;
+    const int lds0 = G > 1 ? grp_id * T::ELEMS : 0;            // the group's part of every stage
     const int col = lane & 31;   // this lane's query within the wavefront
     const int hh = lane >> 5;    // which 8-wide half of an MFMA k-step the lane feeds
-    const int qi = q0 + wave * 32 + col;     // query index within the sequence
+    const int slot = quad * kAttnWaves + wave;
+    const int q0 = slot / per_item * kWaveQ;                 // the wavefront's first query
+    const int head = item * per_item + slot % per_item;
+    const int kvh = (int)(((long long)(item * per_item) * a.n_kv_heads) / a.n_heads);
+    const int qi = q0 + col;                 // query index within the sequence
     const int pos_base = kv_len - q_len;     // absolute position of query 0
     const int qpos = pos_base + qi;
     const bool q_valid = qi < q_len;
 
     // keys this workgroup needs
     int kv_hi = kv_len;
-    if (a.causal) kv_hi = min(kv_len, pos_base + min(q_len, q0 + kBQ));
+    const int q_end = (quad * kAttnWaves + kAttnWaves - 1) / per_item * kWaveQ + kWaveQ;   // past its last query
+    if (a.causal) kv_hi = min(kv_len, pos_base + min(q_len, q_end));
     if (kv_hi < 0) kv_hi = 0;
     const int n_tiles = (kv_hi + kBK - 1) / kBK;
-    const int wave_first_pos = pos_base + q0 + wave * 32;
-    const int wave_last_pos = pos_base + min(q0 + wave * 32 + 31, q_len - 1);
-    const bool wave_has_q = q0 + wave * 32 < q_len;
+    const int wave_first_pos = pos_base + q0;
+    const int wave_last_pos = pos_base + min(q0 + kWaveQ - 1, q_len - 1);
+    const bool wave_has_q = q0 < q_len;
 
     half8 qf[NKK];
     const int hd = NARROW ? a.hd : HD;   // the heads' width in memory
@@ -667,41 +705,81 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_fwd(AttnArgs a) {
     constexpr int kTilePages = kBK / QL_PAGE_SIZE;
     static_assert(kTilePages == kAttnWaves && KvTile<HD>::PAGE_SLOTS == KvTile<HD>::LOADS * kWave,
                   "one page per wavefront");
+    // the group takes tiles grp_id, grp_id + G, ...; every group runs the same number
+    // of steps.  Up to 4 tiles stay with the first group: a prompt of at most 256 keys
+    // gives the same bits at either G, so from the pages as from contiguous rows.
+    const int stride = G > 1 && n_tiles > kOneGroupTiles ? G : 1;
+    const int n_steps = (n_tiles + stride - 1) / stride;
+    auto tile_of = [&](int t) { return G == 1 ? t : stride == G ? G * t + grp_id : grp_id == 0 ? t : n_tiles; };
     WavePagePipe<PAGED> pp;
     pp.init();
     uintptr_t pgk = 0, pgv = 0;   // this wavefront's page of the next tile (paged)
-    if (n_tiles > 0) {
+    if (tile_of(0) < n_tiles) {
         uintptr_t k0 = 0, v0 = 0;
-        pp.entry(a, table, wave);
+        pp.entry(a, table, tile_of(0) * kTilePages + wave);
         pp.pointers(a);
         pp.bases(a, kvh, hd, k0, v0);
-        if (n_tiles > 1) {
-            pp.entry(a, table, kTilePages + wave);
+        if (tile_of(1) < n_tiles) {
+            pp.entry(a, table, tile_of(1) * kTilePages + wave);
             pp.pointers(a);
             pp.bases(a, kvh, hd, pgk, pgv);
         }
-        if (n_tiles > 2) pp.entry(a, table, 2 * kTilePages + wave);
-        load_tile<HD, PAGED, NARROW>(sk0, sv0, a, k0, v0, kvh, 0, kv_len, wave, lane);
+        if (tile_of(2) < n_tiles) pp.entry(a, table, tile_of(2) * kTilePages + wave);
+        load_tile<HD, PAGED, NARROW>(sk0 + lds0, sv0 + lds0, a, k0, v0, kvh, tile_of(0) * kBK, kv_len, wave, lane);
     }
     wait_tile_loads();
     __syncthreads();
-    // tile t sits in (sk, sv); tile t+1 is loaded into (nk, nv) meanwhile
+    // step t's tile sits in (sk, sv); step t+1's is loaded into (nk, nv) meanwhile
     auto step = [&](int t, const _Float16* sk, const _Float16* sv, _Float16* nk, _Float16* nv) {
-        const int kv0 = t * kBK;
-        if (t + 1 < n_tiles) load_tile<HD, PAGED, NARROW>(nk, nv, a, pgk, pgv, kvh, kv0 + kBK, kv_len, wave, lane);
-        if (t + 2 < n_tiles) pp.pointers(a);                                    // tile t+2
-        if (t + 3 < n_tiles) pp.entry(a, table, (t + 3) * kTilePages + wave);   // tile t+3
-        compute(sk, sv, kv0);
-        if (t + 2 < n_tiles) pp.bases(a, kvh, hd, pgk, pgv);
+        if (tile_of(t + 1) < n_tiles)
+            load_tile<HD, PAGED, NARROW>(nk, nv, a, pgk, pgv, kvh, tile_of(t + 1) * kBK, kv_len, wave, lane);
+        if (tile_of(t + 2) < n_tiles) pp.pointers(a);
+        if (tile_of(t + 3) < n_tiles) pp.entry(a, table, tile_of(t + 3) * kTilePages + wave);
+        if (G == 1 || tile_of(t) < n_tiles) compute(sk, sv, tile_of(t) * kBK);
+        if (tile_of(t + 2) < n_tiles) pp.bases(a, kvh, hd, pgk, pgv);
         wait_tile_loads();
         __syncthreads();
     };
-    for (int t = 0; t < n_tiles; t += 2) {
-        step(t, sk0, sv0, sk1, sv1);
-        if (t + 1 >= n_tiles) break;
-        step(t + 1, sk1, sv1, sk0, sv0);
+    for (int t = 0; t < n_steps; t += 2) {
+        step(t, sk0 + lds0, sv0 + lds0, sk1 + lds0, sv1 + lds0);
+        if (t + 1 >= n_steps) break;
+        step(t + 1, sk1 + lds0, sv1 + lds0, sk0 + lds0, sv0 + lds0);
     }
 
+    if constexpr (G > 1) {
+        // the second group's state through the stages (the loop ended on a barrier):
+        // half of its O^T blocks in sk0, half in sv0, (m, l) in sk1
+        static_assert(G == 2 && (size_t)NDB / 2 * 16 * kWave * kAttnWaves * sizeof(float) <= sizeof(sk0), "merge area");
+        float4* ok = reinterpret_cast<float4*>(sk0) + wave * (NDB / 2) * 4 * kWave;
+        float4* ov = reinterpret_cast<float4*>(sv0) + wave * (NDB / 2) * 4 * kWave;
+        float2* ml = reinterpret_cast<float2*>(sk1) + wave * kWave;
+        if (grp_id == 1) {
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                for (int g = 0; g < 4; ++g)
+                    (db < NDB / 2 ? ok : ov)[((db % (NDB / 2)) * 4 + g) * kWave + lane] =
+                        float4{o[db][4 * g], o[db][4 * g + 1], o[db][4 * g + 2], o[db][4 * g + 3]};
+            ml[lane] = float2{m_run, l_run};
+        }
+        __syncthreads();
+        if (grp_id == 1) return;
+        const float2 other = ml[lane];
+        const float m_all = fmaxf(m_run, other.x);
+        const float f0 = __builtin_amdgcn_exp2f((m_run - m_all) * a.cl2);
+        const float f1 = __builtin_amdgcn_exp2f((other.x - m_all) * a.cl2);
+        l_run = fmaf(l_run, f0, other.y * f1);
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const float4 p = (db < NDB / 2 ? ok : ov)[((db % (NDB / 2)) * 4 + g) * kWave + lane];
+                o[db][4 * g] = fmaf(o[db][4 * g], f0, p.x * f1);
+                o[db][4 * g + 1] = fmaf(o[db][4 * g + 1], f0, p.y * f1);
+                o[db][4 * g + 2] = fmaf(o[db][4 * g + 2], f0, p.z * f1);
+                o[db][4 * g + 3] = fmaf(o[db][4 * g + 3], f0, p.w * f1);
+            }
+    }
     if (!q_valid) return;
     store_o<HD>(o, l_run, a.out + (size_t)(q_begin + qi) * a.o_stride + (size_t)head * hd, hh, hd);
 }
@@ -1358,17 +1436,48 @@ float scale_log2e(int head_dim) {
     return (float)((double)scale * 1.4426950408889634);
 }
 
-template <bool PAGED>
-hipError_t launch_attn(const AttnArgs& a, int head_dim, unsigned gx, unsigned gz, hipStream_t stream) {
-    QL_CHECK_ARG((long long)gx * a.n_heads <= INT32_MAX);
-    const dim3 grid(gx * (unsigned)a.n_heads, 1, gz);
+// Whether a prefill of n_wg workgroups over at most max_keys keys runs two wavefront
+// groups a workgroup.  A CU holds two 4-wavefront workgroups or one of 8, so the
+// groups pay while the launch leaves CUs with one 4-wavefront workgroup or none:
+// up to one workgroup a CU; up to two for a causal prompt over its own keys
+// (`triangle`), whose late queries would otherwise be the tail; and a little past one
+// for several sequences, whose longest start first.  Measured on MI355X, 32/8 heads
+// of 128, us at G = 1 / 2 (n_wg): prompt of 256 tokens 11.6 / 11.6 (64), 1000
+// 27.9 / 23.8 (256), 1531 41.1 / 33.8 (384), 2048 56.5 / 49.8 (512), 2560 75.0 / 79.8
+// (640); chunks over 4000 keys of 1024 rows 104 / 81.5 (256), 1300 rows 117 / 121 (328);
+// 512 rows over 8000 keys 197 / 140 (128); 4 x 300 rows over 1767-3000 keys 92 / 77
+// (320); 6 x 250 over 600-1200 keys 45.9 / 49.9 (384).
+constexpr int kCUs = 256;
+
+bool fwd_two_groups(long long n_wg, int n_seqs, bool triangle, long long max_keys) {
+    if (max_keys <= kOneGroupTiles * kBK) return false;
+    return n_wg <= (triangle ? 2 * kCUs : n_seqs > 1 ? kCUs + kCUs / 4 : kCUs);
+}
+
+template <bool PAGED, int G>
+void launch_fwd(const AttnArgs& a, int head_dim, dim3 grid, hipStream_t stream) {
+    const dim3 block(G * kAttnThreads);
     if (head_dim == 128) {
-        hipLaunchKernelGGL((attn_fwd<128, PAGED>), grid, dim3(kAttnThreads), 0, stream, a);
+        hipLaunchKernelGGL((attn_fwd<128, PAGED, false, G>), grid, block, 0, stream, a);
     } else if (head_dim == 64) {
-        hipLaunchKernelGGL((attn_fwd<64, PAGED>), grid, dim3(kAttnThreads), 0, stream, a);
+        hipLaunchKernelGGL((attn_fwd<64, PAGED, false, G>), grid, block, 0, stream, a);
     } else {   // narrow heads, zero-padded to 64 in the tiles
-        hipLaunchKernelGGL((attn_fwd<64, PAGED, true>), grid, dim3(kAttnThreads), 0, stream, a);
+        hipLaunchKernelGGL((attn_fwd<64, PAGED, true, G>), grid, block, 0, stream, a);
     }
+}
+
+// n_seqs sequences of at most max_q_len queries (grid z = sequence).
+template <bool PAGED>
+hipError_t launch_attn(const AttnArgs& a, int head_dim, int max_q_len, unsigned gz, hipStream_t stream) {
+    const int per_item = fwd_heads_per_item(a.n_heads, a.n_kv_heads);
+    const long long quads = ((long long)qlh::blocks_for(max_q_len, kWaveQ) * per_item + kAttnWaves - 1) / kAttnWaves;
+    const long long gx = quads * (a.n_heads / per_item);
+    QL_CHECK_ARG(gx <= INT32_MAX);
+    const dim3 grid((unsigned)gx, 1, gz);
+    const long long max_keys = PAGED ? (long long)a.max_blocks * QL_PAGE_SIZE : a.kv_len;
+    if (fwd_two_groups(gx * gz, (int)gz, !PAGED && a.causal && a.q_len == a.kv_len, max_keys))
+        launch_fwd<PAGED, 2>(a, head_dim, grid, stream);
+    else launch_fwd<PAGED, 1>(a, head_dim, grid, stream);
     return hipGetLastError();
 }
 
@@ -1480,13 +1589,13 @@ extern "C" hipError_t ql_attention_f16(const uint16_t* q, const uint16_t* k, con
     a.v = reinterpret_cast<const _Float16*>(v);
     a.kv_stride = kv_row_stride;
     a.hd = head_dim;
-    if (narrow && q_len > 1) return launch_attn<false>(a, head_dim, qlh::blocks_for(q_len, kBQ), 1, stream);
+    if (narrow && q_len > 1) return launch_attn<false>(a, head_dim, q_len, 1, stream);
     if (!mfma_hd(head_dim) && !narrow) return launch_small<false>(a, q_len, 1, stream);
     if (q_len == 1) {   // decode: the query heads of a KV head share one pass over K/V
         a.n_split = 1;
         return launch_decode<false>(a, head_dim, 1, stream);
     }
-    return launch_attn<false>(a, head_dim, qlh::blocks_for(q_len, kBQ), 1, stream);
+    return launch_attn<false>(a, head_dim, q_len, 1, stream);
 }
 
 extern "C" hipError_t ql_flash_attention_f16(const uint16_t* q, const uint16_t* k,
@@ -1544,7 +1653,7 @@ extern "C" hipError_t ql_paged_attention_f16(
         a.n_split = 1;
         return launch_decode<true>(a, head_dim, n_seqs, stream);
     }
-    return launch_attn<true>(a, head_dim, qlh::blocks_for(max_q_len, kBQ), (unsigned)n_seqs, stream);
+    return launch_attn<true>(a, head_dim, max_q_len, (unsigned)n_seqs, stream);
 }
 
 extern "C" hipError_t ql_paged_decode_workspace_size(int n_seqs, int n_heads, int n_kv_heads,

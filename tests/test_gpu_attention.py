@@ -633,3 +633,60 @@ def test_paged_decode_batch_c5_heads_long_context():
     for s in range(S):
         check_attn(got[s:s + 1], orc.attention(q[s:s + 1], ks[s], vs[s], h, hkv, True, f16=True),
                    vs[s], f"decode seq {s}")
+
+
+# ---- small prefills: two wavefront groups a workgroup ---------------------------------------
+# Contexts beyond 256 keys on few workgroups: the groups split the key tiles (odd and even
+# numbers of them, a last tile of 1 key, early queries whose tiles all stay with the first
+# group), slots of 32 queries over 1, 2, 4, 5 and 8 heads a KV head and heads that do not
+# split evenly, ragged last slots, keys all masked for the second group.
+@pytest.mark.parametrize("h,hkv,d", [(4, 1, 128), (8, 1, 64), (4, 4, 64), (2, 1, 128), (10, 2, 128), (6, 4, 64),
+                                     (16, 8, 40)])
+@pytest.mark.parametrize("q_len,kv_len,causal", [(300, 300, 1), (33, 321, 1), (130, 577, 1), (40, 257, 0), (5, 640, 1)])
+def test_small_prefill_two_groups(h, hkv, d, q_len, kv_len, causal):
+    q = to_f16_bits(normal(h + q_len, (q_len, h, d)))
+    k = to_f16_bits(normal(h + kv_len, (kv_len, hkv, d)))
+    v = to_f16_bits(normal(d + kv_len, (kv_len, hkv, d)))
+    dq, dk, dv = dev(q), dev(k), dev(v)
+    out = Out(q_len * h * d, np.uint16)
+    ql.call("ql_attention_f16", dq.ptr, dk.ptr, dv.ptr, out.ptr, q_len, kv_len, h, hkv, d, h * d, hkv * d, h * d,
+            causal, stream())
+    check_attn(out.get((q_len, h, d)), orc.attention(q, k, v, h, hkv, bool(causal), f16=True), v, "two groups")
+
+
+# Several sequences in one launch, the longest started first whatever their order: equal
+# lengths, a sequence without rows, more sequences than a wavefront has lanes.
+@pytest.mark.parametrize("n_seqs", [3, 64, 70])
+def test_small_paged_prefill_sequence_order(n_seqs):
+    h, hkv, d, L, layer = 2, 1, 64, 2, 1
+    r = np.random.default_rng(n_seqs)
+    ctx = [int(c) for c in r.integers(40, 420, n_seqs)]
+    ctx[1] = ctx[2]
+    qn = [int(min(c, n)) for c, n in zip(ctx, r.integers(1, 50, n_seqs))]
+    qn[0] = 0
+    need = [(c + 15) // 16 for c in ctx]
+    perm = r.permutation(sum(need))
+    tables, o = [], 0
+    for n in need:
+        tables.append(perm[o:o + n])
+        o += n
+    bt = np.full((n_seqs, max(need)), -1, np.int32)
+    for s, t in enumerate(tables):
+        bt[s, :len(t)] = t
+    pool = PagedPool(sum(need), L, hkv, d)
+    ks, vs, qs = [], [], []
+    for s, c in enumerate(ctx):
+        ks.append(to_f16_bits(normal(1000 + s, (c, hkv, d))))
+        vs.append(to_f16_bits(normal(2000 + s, (c, hkv, d))))
+        qs.append(to_f16_bits(normal(3000 + s, (qn[s], h, d))))
+        pool.append(bt[s], ks[s], vs[s], layer)
+    cu = np.concatenate([[0], np.cumsum(qn)]).astype(np.int32)
+    rows = int(cu[-1])
+    dq, dcu, dctx, dbt = dev(np.concatenate(qs)), dev(cu), dev(np.array(ctx, np.int32)), dev(bt)
+    out = Out(rows * h * d, np.uint16)
+    ql.call("ql_paged_attention_f16", dq.ptr, out.ptr, h * d, h * d, rows, n_seqs, dcu.ptr, dctx.ptr, max(qn), dbt.ptr,
+            max(need), pool.kptrs.ptr, pool.vptrs.ptr, pool.nb, layer, L, h, hkv, d, 1, stream())
+    got = out.get((rows, h, d))
+    for s in range(1, n_seqs):
+        want = orc.attention(qs[s], ks[s], vs[s], h, hkv, True, f16=True)
+        check_attn(got[cu[s]:cu[s + 1]], want, vs[s], f"sequence {s} of {n_seqs}")
