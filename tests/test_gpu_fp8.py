@@ -571,3 +571,45 @@ def test_gemm_f16_weight_stream(M, N, K, shift):
     out = empty((M * N,), np.uint16)
     ql.call("ql_gemm_f16", da.ptr + 2 * shift, dw.ptr, out.ptr, M, N, K, stream())
     check_gemm(host(out, shape=(M, N)), gemm_exact(a, w), f"gemm {M}x{N}x{K}")
+
+
+# The tiled GEMM (more than 64 tokens, or fewer with N not a multiple of 16): both tile
+# widths and stage counts (14336 rows), ragged token and weight tiles, odd N (element-wise
+# stores), 2 to 64 steps of 64 k, groups of 1, 2, 5 and 16 steps whose count is and is not
+# a multiple of the four loaded together, K-splits that end inside a group.
+TILE_GEMM_CASES = [
+    (65, 101, 128, ql.QUANT_PER_TENSOR, 0), (129, 1000, 640, ql.QUANT_PER_GROUP, 128),
+    (200, 528, 1024, ql.QUANT_PER_CHANNEL, 0), (332, 96, 4096, ql.QUANT_PER_GROUP, 1024),
+    (130, 264, 2048, ql.QUANT_PER_GROUP, 64), (70, 130, 1600, ql.QUANT_PER_GROUP, 320),
+    (333, 14336, 256, ql.QUANT_PER_GROUP, 128), (512, 14336, 256, ql.QUANT_PER_GROUP, 64),
+    (512, 14336, 192, ql.QUANT_PER_CHANNEL, 0), (96, 64, 4096, ql.QUANT_PER_CHANNEL, 0),
+    (9, 203, 512, ql.QUANT_PER_GROUP, 128), (257, 68, 4032, ql.QUANT_PER_GROUP, 192)]
+
+
+@pytest.mark.parametrize("fmt,mode", [(ql.FP8_E4M3, ql.FP8_MODE_REFERENCE), (ql.FP8_E4M3, ql.FP8_MODE_OCP),
+                                      (ql.FP8_E5M2, ql.FP8_MODE_OCP), (ql.FP8_E5M2, ql.FP8_MODE_REFERENCE)])
+@pytest.mark.parametrize("M,N,K,gran,gs", TILE_GEMM_CASES)
+def test_fp8_gemm_tile(M, N, K, gran, gs, fmt, mode):
+    a = to_f16_bits(normal(5 * M + N + K, (M, K)))
+    w = to_f16_bits(normal(3 * N + K + gs, (N, K), K ** -0.5))
+    q, sc = orc.fp8_quantize(w, fmt, gran, gs, mode)
+    exact = gemm_exact(a, orc.fp8_dequantize(q, sc, fmt, gran, gs, mode))
+    got = gpu_fp8_gemm(a, q, sc, M, N, K, fmt, gran, gs, mode, "query")
+    check_gemm(got, exact, f"fp8 gemm {M}x{N}x{K} gran {gran} gs {gs}")
+
+
+# Codes whose reference decode is not the OCP one, in one row of one tile and one step:
+# that tile is computed again with the checking decoder; in OCP mode a NaN code makes its
+# own weight row NaN and no other.
+@pytest.mark.parametrize("code", [0x01, 0x87, 0x7F])
+@pytest.mark.parametrize("gran,gs", [(ql.QUANT_PER_CHANNEL, 0), (ql.QUANT_PER_GROUP, 128)])
+def test_fp8_gemm_tile_special_codes(code, gran, gs):
+    M, N, K, fmt = 140, 200, 512, ql.FP8_E4M3
+    a = to_f16_bits(normal(code, (M, K)))
+    w = to_f16_bits(normal(code + 1, (N, K), K ** -0.5))
+    for mode in (ql.FP8_MODE_REFERENCE, ql.FP8_MODE_OCP):
+        q, sc = orc.fp8_quantize(w, fmt, gran, gs, mode)
+        q = q.reshape(N, K)
+        q[77, 300] = code
+        exact = gemm_exact(a, orc.fp8_dequantize(q, sc, fmt, gran, gs, mode))
+        check_gemm(gpu_fp8_gemm(a, q, sc, M, N, K, fmt, gran, gs, mode, "query"), exact, f"code {code:#x} mode {mode}")
