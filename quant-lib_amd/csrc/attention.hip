@@ -118,6 +118,8 @@ struct AttnArgs {
     int n_split;                   // key splits per (sequence, KV head)
     float* ws;                     // [n_seqs, n_heads, n_split, head_dim + 2] partials
     int hd;                        // head_dim (read by attn_small and the narrow prefill)
+    // prefill: heads that share an item's key rows, items, quadruples of slots of an item
+    int per_item, n_items, n_quads;
 };
 
 // Page bases of the consecutive 16-key pages of one decode step (up to 4): the
@@ -401,16 +403,13 @@ __device__ __forceinline__ half4 lds_read_tr4(const _Float16* p) {
 // with four heads a KV head its wavefronts hold the same 32 queries and see the same
 // keys: a prompt is padded to 32 rows instead of 128, and no wavefront idles at the
 // causal edge.  (Heads that do not split evenly over the KV heads: one head's slots.)
-__host__ __device__ inline int fwd_heads_per_item(int n_heads, int n_kv_heads) {
-    return n_heads % n_kv_heads == 0 ? n_heads / n_kv_heads : 1;
-}
-
+//
 // KV head (or, ungrouped, query head) and quadruple of slots of a workgroup.
 // Consecutive workgroup ids go to the 8 XCDs in turn; when the heads split evenly
 // over the XCDs, or the XCDs over the heads, each XCD is given its own heads (so
 // their K/V rows stay in that XCD's L2).  Causal: heavy (late) queries first.
-__device__ __forceinline__ void prefill_item(const AttnArgs& a, int n_items, int& item, int& quad) {
-    const int n_quads = (int)gridDim.x / n_items;
+__device__ __forceinline__ void prefill_item(const AttnArgs& a, int& item, int& quad) {
+    const int n_items = a.n_items, n_quads = a.n_quads;
     const int id = (int)blockIdx.x, xcd = id & 7, j = id >> 3;
     int t;
     if (n_items % 8 == 0) {
@@ -563,9 +562,9 @@ __global__ __launch_bounds__(G * kAttnThreads, 2) void attn_fwd(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) _Float16 sk1[G * T::ELEMS];
     __shared__ __attribute__((aligned(16))) _Float16 sv1[G * T::ELEMS];
 
-    const int per_item = fwd_heads_per_item(a.n_heads, a.n_kv_heads);
+    const int per_item = a.per_item;
     int item, quad;
-    prefill_item(a, a.n_heads / per_item, item, quad);
+    prefill_item(a, item, quad);
     int q_begin = 0, q_len = a.q_len, kv_len = a.kv_len;
     const int32_t* table = nullptr;
     if constexpr (PAGED) {
@@ -577,7 +576,9 @@ __global__ __launch_bounds__(G * kAttnThreads, 2) void attn_fwd(AttnArgs a) {
         if (kv_len > a.max_blocks * QL_PAGE_SIZE) kv_len = a.max_blocks * QL_PAGE_SIZE;
         table = a.block_tables + (size_t)s * a.max_blocks;
     }
-    if (quad * kAttnWaves / per_item * kWaveQ >= q_len) return;   // workgroup-uniform
+    // query block and head (of the item's) of the first slot
+    const int block0 = quad * kAttnWaves / per_item, head0 = quad * kAttnWaves - block0 * per_item;
+    if (block0 * kWaveQ >= q_len) return;   // workgroup-uniform
     if (kv_len < 0) kv_len = 0;
 
     const int lane = threadIdx.x & (kWave - 1);
@@ -589,10 +590,23 @@ __global__ __launch_bounds__(G * kAttnThreads, 2) void attn_fwd(AttnArgs a) {
     const int lds0 = G > 1 ? grp_id * T::ELEMS : 0;            // the group's part of every stage
     const int col = lane & 31;   // this lane's query within the wavefront
     const int hh = lane >> 5;    // which 8-wide half of an MFMA k-step the lane feeds
-    const int slot = quad * kAttnWaves + wave;
-    const int q0 = slot / per_item * kWaveQ;                 // the wavefront's first query
-    const int head = item * per_item + slot % per_item;
-    const int kvh = (int)(((long long)(item * per_item) * a.n_kv_heads) / a.n_heads);
+    auto slot = [&](int i, int& block, int& h) {   // slot i (at most 3) of the workgroup's
+        block = block0;
+        h = head0 + i;
+#pragma unroll
+        for (int s = 0; s < kAttnWaves - 1; ++s)
+            if (h >= per_item) {
+                h -= per_item;
+                ++block;
+            }
+    };
+    int q_block, item_head, last_block, last_head;
+    slot(wave, q_block, item_head);
+    slot(kAttnWaves - 1, last_block, last_head);
+    const int q0 = q_block * kWaveQ;                         // the wavefront's first query
+    const int head = item * per_item + item_head;
+    const int kvh = a.n_items == a.n_kv_heads
+                        ? item : (int)((unsigned)item * (unsigned)a.n_kv_heads / (unsigned)a.n_heads);
     const int qi = q0 + col;                 // query index within the sequence
     const int pos_base = kv_len - q_len;     // absolute position of query 0
     const int qpos = pos_base + qi;
@@ -600,8 +614,7 @@ __global__ __launch_bounds__(G * kAttnThreads, 2) void attn_fwd(AttnArgs a) {
 
     // keys this workgroup needs
     int kv_hi = kv_len;
-    const int q_end = (quad * kAttnWaves + kAttnWaves - 1) / per_item * kWaveQ + kWaveQ;   // past its last query
-    if (a.causal) kv_hi = min(kv_len, pos_base + min(q_len, q_end));
+    if (a.causal) kv_hi = min(kv_len, pos_base + min(q_len, (last_block + 1) * kWaveQ));
     if (kv_hi < 0) kv_hi = 0;
     const int n_tiles = (kv_hi + kBK - 1) / kBK;
     const int wave_first_pos = pos_base + q0;
@@ -1468,10 +1481,13 @@ void launch_fwd(const AttnArgs& a, int head_dim, dim3 grid, hipStream_t stream) 
 
 // n_seqs sequences of at most max_q_len queries (grid z = sequence).
 template <bool PAGED>
-hipError_t launch_attn(const AttnArgs& a, int head_dim, int max_q_len, unsigned gz, hipStream_t stream) {
-    const int per_item = fwd_heads_per_item(a.n_heads, a.n_kv_heads);
-    const long long quads = ((long long)qlh::blocks_for(max_q_len, kWaveQ) * per_item + kAttnWaves - 1) / kAttnWaves;
-    const long long gx = quads * (a.n_heads / per_item);
+hipError_t launch_attn(AttnArgs a, int head_dim, int max_q_len, unsigned gz, hipStream_t stream) {
+    a.per_item = a.n_heads % a.n_kv_heads == 0 ? a.n_heads / a.n_kv_heads : 1;
+    a.n_items = a.n_heads / a.per_item;
+    const long long slots = (long long)qlh::blocks_for(max_q_len, kWaveQ) * a.per_item;
+    QL_CHECK_ARG(slots <= INT32_MAX - kAttnWaves);
+    a.n_quads = (int)((slots + kAttnWaves - 1) / kAttnWaves);
+    const long long gx = (long long)a.n_quads * a.n_items;
     QL_CHECK_ARG(gx <= INT32_MAX);
     const dim3 grid((unsigned)gx, 1, gz);
     const long long max_keys = PAGED ? (long long)a.max_blocks * QL_PAGE_SIZE : a.kv_len;
