@@ -456,3 +456,21 @@ def test_engine_layer_c5_shape_prefill_and_decode(prompts):
             b.commit(np.full(plan["n_seqs"], 7, np.int32))
     finally:
         ql.call("ql_engine_destroy", eng)
+
+
+# ---- argmax: rows at every offset from a 16-byte boundary ------------------------------------
+@pytest.mark.parametrize("cols,ld", [(1, 1), (7, 7), (8, 9), (32769, 32771), (65536, 65537), (131073, 131075)])
+@pytest.mark.parametrize("f16", [False, True])
+def test_argmax_any_alignment(cols, ld, f16):
+    rows = 9
+    x = normal(cols + ld, (rows, ld), 3.0)
+    x[:, cols:] = 1e4                        # past the row: never the answer
+    x[1, cols - 1] = x[1, cols // 2] = 60.0  # ties: the first wins
+    x[2, 0] = 60.0
+    x[3, cols - 1] = 60.0
+    xb = to_f16_bits(x) if f16 else x
+    want = orc.argmax((f16_bits_to_f32(xb) if f16 else xb)[:, :cols])
+    d = dev(np.ascontiguousarray(xb).reshape(-1))
+    out = empty((rows,), np.int32)
+    ql.call("ql_argmax_f16" if f16 else "ql_argmax_f32", d.ptr, rows, cols, ld, out.ptr, stream())
+    assert list(host(out)) == list(want)
