@@ -1112,11 +1112,13 @@ __device__ __forceinline__ bool dec_sequence(const AttnArgs& a, int s, int& q_ro
 
 // NARROW: contiguous K/V with heads of a.hd < 64 (a multiple of 8) on the HD 64
 // kernel, zero-padded, one key split.
-template <int HD, bool PAGED, bool NARROW = false>
+// SORTED: the sequences start longest first (more workgroups than run at once).
+template <int HD, bool PAGED, bool NARROW = false, bool SORTED = false>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_decode(AttnArgs a) {
     using T = Dec<HD>;
     __shared__ __attribute__((aligned(16))) char smem_raw[T::SMEM_BYTES];
-    const int s = blockIdx.z, kvh = blockIdx.y;
+    const int s = SORTED ? longest_first(a.ctx_lens, (int)gridDim.z, (int)blockIdx.z) : (int)blockIdx.z;
+    const int kvh = blockIdx.y;
     const int sp = (int)blockIdx.x % a.n_split, cg = (int)blockIdx.x / a.n_split;
     // query heads h with h*n_kv_heads/n_heads == kvh: [ceil(kvh*H/Hkv), ceil((kvh+1)*H/Hkv))
     const long long H = a.n_heads, HK = a.n_kv_heads;
@@ -1547,15 +1549,21 @@ size_t dec_ws_bytes(int n_seqs, int n_heads, int head_dim, int n_split) {
 template <bool PAGED>
 hipError_t launch_decode(const AttnArgs& a, int head_dim, int n_seqs, hipStream_t stream) {
     const int n_cg = dec_col_chunks(a.n_heads, a.n_kv_heads);
+    // past two workgroups a CU the last ones should be short: 48 sequences of 2048-4096
+    // keys, 32/8 heads of 128 (768 workgroups) 123.7 -> 118.7 us on MI355X; with more
+    // than two splits a sequence they are already (20 x 13000 keys: 157.4 -> 158.4)
+    const bool sorted = PAGED && n_seqs > 1 && a.n_split <= 2 && (long long)n_seqs * a.n_kv_heads * n_cg * a.n_split > 2 * kCUs;
     QL_CHECK_ARG((long long)a.n_split * n_cg <= INT32_MAX);
     const dim3 grid((unsigned)(a.n_split * n_cg), (unsigned)a.n_kv_heads, (unsigned)n_seqs);
     const dim3 cgrid((unsigned)a.n_heads, (unsigned)n_seqs);
     if (head_dim == 128) {
-        hipLaunchKernelGGL((attn_decode<128, PAGED>), grid, dim3(kAttnThreads), 0, stream, a);
+        if (sorted) hipLaunchKernelGGL((attn_decode<128, PAGED, false, PAGED>), grid, dim3(kAttnThreads), 0, stream, a);
+        else hipLaunchKernelGGL((attn_decode<128, PAGED>), grid, dim3(kAttnThreads), 0, stream, a);
         if (a.n_split > 1)
             hipLaunchKernelGGL((attn_decode_combine<128, PAGED>), cgrid, dim3(kMaxSplits), 0, stream, a);
     } else if (head_dim == 64) {
-        hipLaunchKernelGGL((attn_decode<64, PAGED>), grid, dim3(kAttnThreads), 0, stream, a);
+        if (sorted) hipLaunchKernelGGL((attn_decode<64, PAGED, false, PAGED>), grid, dim3(kAttnThreads), 0, stream, a);
+        else hipLaunchKernelGGL((attn_decode<64, PAGED>), grid, dim3(kAttnThreads), 0, stream, a);
         if (a.n_split > 1)
             hipLaunchKernelGGL((attn_decode_combine<64, PAGED>), cgrid, dim3(kMaxSplits), 0, stream, a);
     } else {   // narrow heads: one split (the caller sets n_split = 1)

@@ -690,3 +690,32 @@ def test_small_paged_prefill_sequence_order(n_seqs):
     for s in range(1, n_seqs):
         want = orc.attention(qs[s], ks[s], vs[s], h, hkv, True, f16=True)
         check_attn(got[cu[s]:cu[s + 1]], want, vs[s], f"sequence {s} of {n_seqs}")
+
+
+def test_paged_decode_longest_first():
+    # more workgroups than run at once (70 x 8 KV heads): sequences of very different
+    # lengths, in the order of their lengths or (beyond 64 sequences) of their numbers
+    for n_seqs in (40, 64, 70):
+        h, hkv, d, L, layer = 16, 16, 64, 1, 0
+        r = np.random.default_rng(n_seqs)
+        ctx = [int(c) for c in r.integers(1, 300, n_seqs)]
+        need = [(c + 15) // 16 for c in ctx]
+        perm = r.permutation(sum(need))
+        bt = np.full((n_seqs, max(need)), -1, np.int32)
+        pool = PagedPool(sum(need), L, hkv, d)
+        ks, vs, o = [], [], 0
+        for s, c in enumerate(ctx):
+            bt[s, :need[s]] = perm[o:o + need[s]]
+            o += need[s]
+            ks.append(to_f16_bits(normal(100 + s, (c, hkv, d))))
+            vs.append(to_f16_bits(normal(200 + s, (c, hkv, d))))
+            pool.append(bt[s], ks[s], vs[s], layer)
+        qs = to_f16_bits(normal(n_seqs, (n_seqs, h, d)))
+        dq, dctx, dbt = dev(qs), dev(np.array(ctx, np.int32)), dev(bt)
+        out = Out(n_seqs * h * d, np.uint16)
+        ql.call("ql_paged_decode_attention_f16", dq.ptr, out.ptr, h * d, h * d, n_seqs, dctx.ptr, max(ctx), dbt.ptr,
+                max(need), pool.kptrs.ptr, pool.vptrs.ptr, pool.nb, layer, L, h, hkv, d, None, 0, stream())
+        got = out.get((n_seqs, h, d))
+        for s in range(n_seqs):
+            want = orc.attention(qs[s:s + 1], ks[s], vs[s], h, hkv, True, f16=True)
+            check_attn(got[s:s + 1], want, vs[s], f"sequence {s} of {n_seqs}")
