@@ -270,26 +270,108 @@ __global__ void finalize_scales(float* __restrict__ s, int n, float fmax) {
 }
 
 // ---- quantize / dequantize ------------------------------------------------------------
-// 8 elements times their group's scale -> 8 codes (s: one float, or one per element)
+// Four scaled values -> the reference encoder's four codes; none of them is a NaN.
+// enc_ref clamps and truncates, so on the high halves of the fp32 words (sign,
+// exponent, 7 bits of fraction) it is a shift, a minimum with the code of the
+// largest value, a saturating subtraction of the exponent bias that also takes the
+// codes of exponent 0 to zero, and two 16-bit lanes do it at once: about 5
+// instructions an element instead of 15.
+typedef uint16_t ushort2v __attribute__((ext_vector_type(2)));
+template <int FMT>
+__device__ __forceinline__ uint32_t enc_ref4(const float (&f)[4]) {
+    constexpr int MB = FMT == QL_FP8_E4M3 ? 3 : 2, BIAS = FMT == QL_FP8_E4M3 ? 7 : 15;
+    constexpr uint16_t kFrac = (1 << MB) - 1;                    // largest code of exponent 0
+    constexpr uint16_t kBase = (127 - BIAS) << MB;               // shifted word of code 0
+    constexpr uint16_t kTop = kBase + (FMT == QL_FP8_E4M3 ? 0x7E : 0x7B);
+    uint32_t h[2], c[2];
+    uint32_t one = 0x00010001u, frac = kFrac * 0x00010001u;   // unknown to the compiler: it makes two
+    asm("" : "+s"(one), "+s"(frac));                           // compares and selects of a minimum with 1
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        h[p] = __builtin_amdgcn_perm(__float_as_uint(f[2 * p + 1]), __float_as_uint(f[2 * p]), 0x07060302u);
+        ushort2v t = __builtin_bit_cast(ushort2v, h[p] & 0x7FFF7FFFu) >> (uint16_t)(7 - MB);
+        t = __builtin_elementwise_min(t, (ushort2v)kTop);
+        t = __builtin_elementwise_sub_sat(t, (ushort2v)(uint16_t)(kBase + kFrac));   // code - kFrac, 0 below
+        t += __builtin_elementwise_min(t, __builtin_bit_cast(ushort2v, one)) * __builtin_bit_cast(ushort2v, frac);
+        c[p] = __builtin_bit_cast(uint32_t, t);
+    }
+    return __builtin_amdgcn_perm(c[1], c[0], 0x06040200u) |
+           (__builtin_amdgcn_perm(h[1], h[0], 0x07050301u) & 0x80808080u);
+}
+
+// 8 elements times their group's scale -> 8 codes (s: one float, or one per element).
+// A lane with a NaN among its scaled elements takes the one-element encoders.
 template <int FMT, int MODE, typename S = float>
 __device__ __forceinline__ u32x2 encode8(const Vec<_Float16, 8>& v, const S& s) {
+    constexpr float fm = fp8_max(FMT);
+    float f[2][4];
+    bool nan = false;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        if constexpr (std::is_same_v<S, float>) f[e >> 2][e & 3] = (float)v.v[e] * s;
+        else f[e >> 2][e & 3] = (float)v.v[e] * s[e];
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e += 2) nan |= __builtin_isunordered(f[e >> 2][e & 3], f[e >> 2][(e & 3) + 1]);
     uint32_t w[2];
+    if (nan) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if constexpr (MODE == QL_FP8_MODE_REFERENCE)
+                w[h] = enc_ref<FMT>(f[h][0]) | (enc_ref<FMT>(f[h][1]) << 8) | (enc_ref<FMT>(f[h][2]) << 16) |
+                       (enc_ref<FMT>(f[h][3]) << 24);
+            else
+                w[h] = enc_ocp2<FMT>(f[h][0], f[h][1]) | (enc_ocp2<FMT>(f[h][2], f[h][3]) << 16);
+        }
+        return u32x2{w[0], w[1]};
+    }
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-        float f[4];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            if constexpr (std::is_same_v<S, float>) f[e] = (float)v.v[4 * h + e] * s;
-            else f[e] = (float)v.v[4 * h + e] * s[4 * h + e];
-        }
         if constexpr (MODE == QL_FP8_MODE_REFERENCE) {
-            w[h] = enc_ref<FMT>(f[0]) | (enc_ref<FMT>(f[1]) << 8) | (enc_ref<FMT>(f[2]) << 16) |
-                   (enc_ref<FMT>(f[3]) << 24);
+            w[h] = enc_ref4<FMT>(f[h]);
         } else {
-            w[h] = enc_ocp2<FMT>(f[0], f[1]) | (enc_ocp2<FMT>(f[2], f[3]) << 16);
+            float c[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) c[e] = __builtin_amdgcn_fmed3f(f[h][e], -fm, fm);
+            int lo, both;
+            if constexpr (FMT == QL_FP8_E4M3) {
+                lo = __builtin_amdgcn_cvt_pk_fp8_f32(c[0], c[1], 0, false);
+                both = __builtin_amdgcn_cvt_pk_fp8_f32(c[2], c[3], lo, true);
+            } else {
+                lo = __builtin_amdgcn_cvt_pk_bf8_f32(c[0], c[1], 0, false);
+                both = __builtin_amdgcn_cvt_pk_bf8_f32(c[2], c[3], lo, true);
+            }
+            w[h] = (uint32_t)both;
         }
     }
     return u32x2{w[0], w[1]};
+}
+
+// the largest |x| of 8 elements (NaNs left out), two at a time in binary16: the
+// maximum is one of them, so no rounding enters
+__device__ __forceinline__ float absmax8(const Vec<_Float16, 8>& v) {
+    const u32x4 w = __builtin_bit_cast(u32x4, v);
+    half2v m = {0, 0};
+#pragma unroll
+    for (int p = 0; p < 4; ++p) m = __builtin_elementwise_max(m, __builtin_bit_cast(half2v, w[p] & 0x7FFF7FFFu));
+    return fmaxf((float)m[0], (float)m[1]);
+}
+
+// the maximum over aligned groups of GL lanes, in every lane of the group: inside a
+// row of 16 lanes from DPP moves (each step mirrors onto the half not yet taken in)
+template <int CTRL>
+__device__ __forceinline__ float max_dpp(float v) {
+    return fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true)));
+}
+template <int GL>
+__device__ __forceinline__ float group_max(float m) {
+    if constexpr (GL >= 2) m = max_dpp<0xB1>(m);    // quad_perm 1,0,3,2
+    if constexpr (GL >= 4) m = max_dpp<0x4E>(m);    // quad_perm 2,3,0,1
+    if constexpr (GL >= 8) m = max_dpp<0x141>(m);   // row_half_mirror
+    if constexpr (GL >= 16) m = max_dpp<0x140>(m);  // row_mirror
+#pragma unroll
+    for (int o = 16; o < GL; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, kWave));
+    return m;
 }
 
 // The scales of the 8 elements from e0 (a multiple of 8): groups that are not a
@@ -343,6 +425,9 @@ __global__ __launch_bounds__(kBlock) void quantize_kernel(const _Float16* __rest
 // group's scale exactly as finalize_scales does (fmax / max, 1 below 1e-8) and
 // encodes its 8 elements from the registers it loaded, so x is read once instead
 // of twice.  One lane per group stores the scale.
+// Bound by HBM (3 bytes an element) once the encoder takes 5 instructions an element
+// and the group's maximum DPP moves: 14336 x 4096 in groups of 128, reference codec,
+// 43 -> 31.5 us (5.6 TB/s, what a copy of its size reaches); the codes are unchanged.
 constexpr int kQuantIters = 4;   // spans of 64 vectors per wavefront (2, 4, 8, 16 measured: 4 best)
 
 template <int FMT, int MODE, int GL>
@@ -362,13 +447,8 @@ __global__ __launch_bounds__(kBlock) void quantize_groups(const _Float16* __rest
     for (int it = 0; it < kQuantIters; ++it) {
         const long long v = w0 + (long long)it * kWave + lane;
         const long long off = (v * 8) % (8 * GL);                 // offset inside the group
-        float m = 0.0f;   // lanes past the end (their load repeated vector 0) add nothing
-        if (v < n_vec && seen(MODE, off)) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf((float)h[it].v[e]));
-        }
-#pragma unroll
-        for (int o = 1; o < GL; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, kWave));
+        // lanes past the end (their load repeated vector 0) add nothing
+        const float m = group_max<GL>(v < n_vec && seen(MODE, off) ? absmax8(h[it]) : 0.0f);
         const float sc = m < 1e-8f ? 1.0f : kMax / m;
         if (v < n_vec) {
             if ((lane & (GL - 1)) == 0) scales[v / GL] = sc;
@@ -404,11 +484,7 @@ __global__ __launch_bounds__(kBlock) void quantize_segments(const _Float16* __re
     for (int it = 0; it < kQuantIters; ++it) {
         const long long v = (sp0 + it) * P * V + lane;
         const bool ok = in_span && v < n_vec;
-        float m = 0.0f;
-        if (ok && seen(MODE, (long long)idx * 8)) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf((float)h[it].v[e]));
-        }
+        float m = ok && seen(MODE, (long long)idx * 8) ? absmax8(h[it]) : 0.0f;
         for (int o = 1; o < V; o <<= 1) {   // uniform trip count
             const float t = __shfl(m, min(lane + o, kWave - 1), kWave);
             if (idx + o < V) m = fmaxf(m, t);
@@ -457,10 +533,7 @@ __global__ __launch_bounds__(WPG == 1 ? kBlock : kWave * WPG) void quantize_wave
 #pragma unroll
     for (int j = 0; j < NV; ++j) {
         const int i = j * kSpan + off;
-        if (i < nv && seen(MODE, (long long)i * 8)) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf((float)h[j].v[e]));
-        }
+        if (i < nv && seen(MODE, (long long)i * 8)) m = fmaxf(m, absmax8(h[j]));
     }
     m = wave_max(m);
     if constexpr (WPG > 1) {
@@ -515,39 +588,77 @@ __device__ __forceinline__ void decode4(uint32_t w, float (&d)[4]) {
     }
 }
 
-// 16 codes per thread (n % 16 == 0, gs % 16 == 0, 16-byte aligned codes and output):
-// one 16-byte load, the group's scale and its reciprocal once, two 16-byte stores.
+// 8 codes of one group -> binary16(decode(code) / s).  The hardware decodes four
+// codes in two instructions, and a lane whose codes are all finite and decode alike in
+// both conventions needs no test on an element: the correction of div_by_recip takes
+// a zero to +0, which is the reference's value of both its zero codes and, with the
+// code's sign put back, the OCP one.  Other lanes decode and test one by one.
 template <int FMT, int MODE>
-__global__ __launch_bounds__(kBlock) void dequantize16(const uint8_t* __restrict__ q, Geom g,
-                                                       const float* __restrict__ scales,
-                                                       _Float16* __restrict__ y) {
-    const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (t * 16 >= g.n) return;
-    const u32x4 w = load<true>(reinterpret_cast<const u32x4*>(q) + t);
-    const long long e0 = t * 16;
-    const long long gi = g.n <= 0xFFFFFFFFLL ? (long long)((uint32_t)e0 / (uint32_t)g.gs) : e0 / g.gs;
-    const float s = scales[gi];
-    Vec<_Float16, 8> out[2];
-    if (recip_ok(s)) {
-        const float r = 1.0f / s;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float d[4];
-            decode4<FMT, MODE>(w[j], d);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) out[j >> 1].v[4 * (j & 1) + e] = from_f32<_Float16>(div_by_recip(d[e], s, r));
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            float d[4];
-            decode4<FMT, MODE>(w[j], d);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) out[j >> 1].v[4 * (j & 1) + e] = from_f32<_Float16>(d[e] / s);
-        }
+__device__ __forceinline__ Vec<_Float16, 8> dequantize8(u32x2 w, float s) {
+    Vec<_Float16, 8> out;
+    uint32_t special;
+    if constexpr (MODE == QL_FP8_MODE_REFERENCE) {
+        special = ref_special<FMT>(w[0]) | ref_special<FMT>(w[1]);
+    } else {   // infinities and NaNs
+        constexpr uint32_t kTop = FMT == QL_FP8_E4M3 ? 0x01010101u : 0x04040404u;
+        special = ((w[0] & 0x7F7F7F7Fu) + kTop) | ((w[1] & 0x7F7F7F7Fu) + kTop);
     }
-    store<true>(reinterpret_cast<Vec<_Float16, 8>*>(y) + 2 * t, out[0]);
-    store<true>(reinterpret_cast<Vec<_Float16, 8>*>(y) + 2 * t + 1, out[1]);
+    const float r = 1.0f / s;
+    if (recip_ok(s) && !(special & 0x80808080u)) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const float2v lo = dec_ocp2<FMT>(w[j]), hi = dec_ocp2<FMT, true>(w[j]);
+            const float d[4] = {lo[0], lo[1], hi[0], hi[1]};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float q0 = d[e] * r;
+                float q1 = fmaf(fmaf(-q0, s, d[e]), r, q0);
+                if constexpr (MODE != QL_FP8_MODE_REFERENCE) q1 = copysignf(q1, d[e]);
+                out.v[4 * j + e] = from_f32<_Float16>(q1);
+            }
+        }
+        return out;
+    }
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        float d[4];
+        decode4<FMT, MODE>(w[j], d);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            out.v[4 * j + e] = from_f32<_Float16>(recip_ok(s) ? div_by_recip(d[e], s, r) : d[e] / s);
+    }
+    return out;
+}
+
+// Groups of a multiple of 8 codes (n % 8 == 0, 8-byte aligned codes, 16-byte aligned
+// output): kDequantIters vectors of 8 codes a thread, a workgroup's width apart, so
+// that each store instruction of a wavefront writes 64 vectors that follow one another
+// (16 codes a thread and two stores 32 bytes apart wrote every line in two halves).
+// Bound by HBM, 3 bytes a code: 14336 x 4096 in groups of 128, reference codec,
+// 36 -> 30 us (5.9 TB/s); the values are unchanged.
+constexpr int kDequantIters = 4;
+
+template <int FMT, int MODE>
+__global__ __launch_bounds__(kBlock) void dequantize_groups(const uint8_t* __restrict__ q, Geom g, int gs_shift,
+                                                            const float* __restrict__ scales,
+                                                            _Float16* __restrict__ y) {
+    const long long v0 = (long long)blockIdx.x * (kDequantIters * kBlock) + threadIdx.x;
+    const long long n_vec = g.n / 8;
+    u32x2 w[kDequantIters];
+    float s[kDequantIters];
+#pragma unroll
+    for (int it = 0; it < kDequantIters; ++it) {   // every load first; past the end vector 0
+        const long long v = v0 + it * kBlock < n_vec ? v0 + it * kBlock : 0;
+        w[it] = load<true>(reinterpret_cast<const u32x2*>(q) + v);
+        const long long e0 = v * 8;
+        s[it] = scales[gs_shift >= 0 ? e0 >> gs_shift   // uniform
+                       : g.n <= 0xFFFFFFFFLL ? (long long)((uint32_t)e0 / (uint32_t)g.gs) : e0 / g.gs];
+    }
+#pragma unroll
+    for (int it = 0; it < kDequantIters; ++it) {
+        const long long v = v0 + it * kBlock;
+        if (v < n_vec) store<true>(reinterpret_cast<Vec<_Float16, 8>*>(y) + v, dequantize8<FMT, MODE>(w[it], s[it]));
+    }
 }
 
 template <int FMT, int MODE, bool VEC>
@@ -559,44 +670,29 @@ __global__ __launch_bounds__(kBlock) void dequantize_kernel(const uint8_t* __res
         if (t * 8 >= g.n) return;
         const u32x2 w = load<true>(reinterpret_cast<const u32x2*>(q) + t);
         Vec<_Float16, 8> out;
-        if (g.gs % 8) {   // uniform: groups start inside vectors
-            float s8[8];
-            scales8(scales, g, t * 8, s8);
-            bool ok = true;
+        float s8[8];
+        scales8(scales, g, t * 8, s8);
+        bool ok = true;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) ok = ok && recip_ok(s8[e]);
-            if (ok) {   // both forms give RN(d / s); at most 2 distinct scales when gs >= 8
-                float r8[8];
-                if (g.gs >= 8) {   // s8 holds the scales of at most two groups, in order
-                    const float ra = 1.0f / s8[0], rb = 1.0f / s8[7];
+        for (int e = 0; e < 8; ++e) ok = ok && recip_ok(s8[e]);
+        if (ok) {   // both forms give RN(d / s); at most 2 distinct scales when gs >= 8
+            float r8[8];
+            if (g.gs >= 8) {   // s8 holds the scales of at most two groups, in order
+                const float ra = 1.0f / s8[0], rb = 1.0f / s8[7];
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) r8[e] = s8[e] == s8[0] ? ra : rb;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) r8[e] = 1.0f / s8[e];
-                }
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    out.v[e] = from_f32<_Float16>(
-                        div_by_recip(decode1<FMT, MODE>((w[e >> 2] >> (8 * (e & 3))) & 0xFFu), s8[e], r8[e]));
+                for (int e = 0; e < 8; ++e) r8[e] = s8[e] == s8[0] ? ra : rb;
             } else {
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    out.v[e] = from_f32<_Float16>(decode1<FMT, MODE>((w[e >> 2] >> (8 * (e & 3))) & 0xFFu) / s8[e]);
+                for (int e = 0; e < 8; ++e) r8[e] = 1.0f / s8[e];
             }
-            store<true>(reinterpret_cast<Vec<_Float16, 8>*>(y) + t, out);
-            return;
-        }
-        const float s = scales[(t * 8) / g.gs];
-        if (recip_ok(s)) {
-            const float r = 1.0f / s;
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                out.v[e] = from_f32<_Float16>(div_by_recip(decode1<FMT, MODE>((w[e >> 2] >> (8 * (e & 3))) & 0xFFu), s, r));
+                out.v[e] = from_f32<_Float16>(
+                    div_by_recip(decode1<FMT, MODE>((w[e >> 2] >> (8 * (e & 3))) & 0xFFu), s8[e], r8[e]));
         } else {
 #pragma unroll
             for (int e = 0; e < 8; ++e)
-                out.v[e] = from_f32<_Float16>(decode1<FMT, MODE>((w[e >> 2] >> (8 * (e & 3))) & 0xFFu) / s);
+                out.v[e] = from_f32<_Float16>(decode1<FMT, MODE>((w[e >> 2] >> (8 * (e & 3))) & 0xFFu) / s8[e]);
         }
         store<true>(reinterpret_cast<Vec<_Float16, 8>*>(y) + t, out);
     } else {
@@ -1471,9 +1567,11 @@ void launch_quantize(const _Float16* x, const Geom& g, const float* s, uint8_t* 
 template <int FMT, int MODE>
 void launch_dequantize(const uint8_t* q, const Geom& g, const float* s, _Float16* y, bool vec,
                        hipStream_t st) {
-    if (vec && g.n % 16 == 0 && g.gs % 16 == 0 && qlh::aligned16(q))
-        hipLaunchKernelGGL((dequantize16<FMT, MODE>), dim3(qlh::blocks_for(g.n / 16, kBlock)), dim3(kBlock), 0,
-                           st, q, g, s, y);
+    const int shift = (g.gs & (g.gs - 1)) == 0 ? __builtin_ctzll((unsigned long long)g.gs) : -1;
+    if (vec && g.gs % 8 == 0)
+        hipLaunchKernelGGL((dequantize_groups<FMT, MODE>),
+                           dim3(qlh::blocks_for(g.n / 8, (long long)kDequantIters * kBlock)), dim3(kBlock), 0, st,
+                           q, g, shift, s, y);
     else if (vec)
         hipLaunchKernelGGL((dequantize_kernel<FMT, MODE, true>), dim3(qlh::blocks_for(g.n / 8, kBlock)),
                            dim3(kBlock), 0, st, q, g, s, y);

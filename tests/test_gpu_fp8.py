@@ -157,8 +157,7 @@ def test_fp8_dequantize_any_scale_bit_exact(mode, fmt, gs):
     # every code under log-uniform scales from 2^-100 to 2^100 (the dequantizer divides
     # by a corrected reciprocal for scales in [2^-90, 2^90] and by fp32 division
     # outside), plus scales at and just past those limits: bit for bit the oracle's
-    # binary16(decode / scale), NaN for NaN.  Groups of 32 take the 16-codes-per-thread
-    # kernel, groups of 8 the 8-codes one.
+    # binary16(decode / scale), NaN for NaN.
     rng = np.random.default_rng(40 + 2 * fmt + mode)
     n_grp = 2048
     edges = np.array([2.0 ** -90, 2.0 ** 90, np.nextafter(np.float32(2.0 ** -90), 0),
@@ -170,6 +169,32 @@ def test_fp8_dequantize_any_scale_bit_exact(mode, fmt, gs):
     got = gpu_dequantize(codes, scg, fmt, ql.QUANT_PER_GROUP, gs, mode)
     want = orc.fp8_dequantize(codes, scg, fmt, ql.QUANT_PER_GROUP, gs, mode)
     assert same_f16(got, want), int((got != want).sum())
+
+
+@pytest.mark.parametrize("rows,cols,gran,gs", [
+    (1, 8, ql.QUANT_PER_GROUP, 8), (3, 2728, ql.QUANT_PER_GROUP, 88),    # one vector; the last one of a 2nd workgroup
+    (33, 1000, ql.QUANT_PER_GROUP, 40), (64, 960, ql.QUANT_PER_GROUP, 24), (16, 512, ql.QUANT_PER_GROUP, 16),
+    (5, 1016, ql.QUANT_PER_CHANNEL, 0), (7, 6152, ql.QUANT_PER_CHANNEL, 0), (9, 904, ql.QUANT_PER_TENSOR, 0)])
+@pytest.mark.parametrize("mode", MODES)
+@pytest.mark.parametrize("fmt", FMTS)
+def test_fp8_codec_mixed_special_vectors(mode, fmt, rows, cols, gran, gs):
+    # vectors of 8 with and without a NaN (quiet and signalling, both signs), values far
+    # above the scale's range (infinite once scaled), signed zeros and subnormals; then
+    # every code, so that vectors with and without the codes decoded one by one mix
+    rng = np.random.default_rng(rows + cols)
+    x = to_f16_bits(uniform(rows * cols, (rows, cols), -1.0, 1.0))
+    at = rng.random((rows, cols)) < 0.06
+    odd = np.array([0x7E00, 0xFE01, 0x7C01, 0xFDFF, 0x7BFF, 0xFBFF, 0x0000, 0x8000, 0x0001, 0x8003, 0x03FF], np.uint16)
+    x[at] = rng.choice(odd, int(at.sum()))
+    x[:, :4] = to_f16_bits(np.full((rows, 4), 0.5, np.float32))
+    q, sc = gpu_quantize(x, fmt, gran, gs, mode)
+    # the oracle sees quiet NaNs: fmaxf of the C library turns a signalling one into its result
+    q_want, sc_want = orc.fp8_quantize(np.where((x & 0x7FFF) > 0x7C00, x | 0x0200, x), fmt, gran, gs, mode)
+    assert np.array_equal(sc, sc_want)
+    assert np.array_equal(q, q_want), int((q != q_want).sum())
+    codes = rng.integers(0, 256, (rows, cols)).astype(np.uint8)
+    codes[rng.random((rows, cols)) < 0.9] = 0x80
+    assert same_f16(gpu_dequantize(codes, sc, fmt, gran, gs, mode), orc.fp8_dequantize(codes, sc, fmt, gran, gs, mode))
 
 
 def gemm_exact(a, w_deq):
