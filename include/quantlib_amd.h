@@ -443,8 +443,10 @@ hipError_t ql_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, int M,
  * over copies of >= 512 MB in total, so they stream from HBM as in a multi-layer
  * step).  The fastest four are re-timed with the heuristic's first choice in three
  * alternating rounds, and the first choice is kept unless one of them is more than
- * 3% faster over those rounds.  Setup only: allocates and frees scratch, synchronizes `stream`, and must
- * not run under graph capture.  Later ql_gemm_f16 calls of that shape use the
+ * 3% faster over those rounds.  Where ql_gemm_f16 takes few rows to its own kernel
+ * instead of the library, that kernel is timed in the same rounds and stays unless
+ * the library is more than 3% faster.  Setup only: allocates and frees scratch,
+ * synchronizes `stream`, and must not run under graph capture.  Later ql_gemm_f16 calls of that shape use the
  * chosen algorithm; results stay within the GEMM's fp32-accumulation tolerance
  * but may differ in the last bits from the untuned plan.  No counterpart in the
  * reference (its cuBLAS calls take the library default). */

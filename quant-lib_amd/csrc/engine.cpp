@@ -189,7 +189,7 @@ hipError_t layer_forward(ql_engine* e, const uint16_t* attn_norm, const uint16_t
     if (s->n_seqs == 1 && s->max_q_len == T && s->max_ctx_len == T && T > 1) {
         // one fresh prompt: its keys are exactly this step's rows, still in the QKV
         // buffer (rotated in place), so the contiguous kernel reads them through the
-        // row stride instead of the pool (same arithmetic, no page lookups)
+        // row stride instead of the pool (no page lookups)
         QL_TRY(ql_attention_f16(q, k, v, e->attn, T, T, H, HK, HD, QKV, QKV, (int64_t)H * HD, 1, stream));
     } else if (s->max_q_len == 1 && T == s->n_seqs) {   // every sequence decodes: row i = sequence i
         QL_TRY(ql_paged_decode_attention_f16(q, e->attn, QKV, (int64_t)H * HD, s->n_seqs, s->ctx_lens,

@@ -30,6 +30,7 @@ struct Plan {
     hipblasLtMatmulDesc_t desc = nullptr;
     hipblasLtMatrixLayout_t a = nullptr, b = nullptr, c = nullptr;
     hipblasLtMatmulAlgo_t algo{};
+    bool over_stream = false;   // tuned, and faster than the weight-stream kernel
 };
 
 struct Device {
@@ -87,6 +88,15 @@ hipError_t make_plan(Device& d, int M, int N, int K, Plan& p) {
     return hipSuccess;
 }
 
+// Whether ql_gemm_tune_f16 found the library faster than the weight-stream kernel.
+bool tuned_to_library(int dev, int M, int N, int K) {
+    std::lock_guard<std::mutex> lock(g_mu);
+    const auto d = g_devices.find(dev);
+    if (d == g_devices.end()) return false;
+    const auto it = d->second.plans.find(std::make_tuple(M, N, K));
+    return it != d->second.plans.end() && it->second.over_stream;
+}
+
 }  // namespace
 
 extern "C" hipError_t ql_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int N,
@@ -94,9 +104,10 @@ extern "C" hipError_t ql_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t
     if (M < 0 || N < 0 || K < 0) return hipErrorInvalidValue;
     if (M == 0 || N == 0) return hipSuccess;
     if (!x || !w || !y || K == 0) return hipErrorInvalidValue;
-    if (qlh::stream_gemm_f16_applies(x, w, M, N, K)) return qlh::stream_gemm_f16(x, w, y, M, N, K, stream);
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return hipErrorNoDevice;
+    if (qlh::stream_gemm_f16_applies(x, w, M, N, K) && !tuned_to_library(dev, M, N, K))
+        return qlh::stream_gemm_f16(x, w, y, M, N, K, stream);
     Plan plan;
     void* ws = nullptr;
     hipblasLtHandle_t lt = nullptr;
@@ -190,15 +201,19 @@ extern "C" hipError_t ql_gemm_tune_f16(int M, int N, int K, hipStream_t stream) 
     if ((e = hipMemsetAsync(xs.p, 0x11, xb, stream)) != hipSuccess) return e;
     if ((e = hipMemsetAsync(ws_.p, 0x11, wb * (size_t)copies, stream)) != hipSuccess) return e;
     const float alpha = 1.0f, beta = 0.0f;
-    auto run = [&](const hipblasLtMatmulAlgo_t& algo, int i) {
+    // algo null: the weight-stream kernel
+    auto run = [&](const hipblasLtMatmulAlgo_t* algo, int i) {
         const char* w = static_cast<const char*>(ws_.p) + (size_t)(i % copies) * wb;
+        if (!algo)
+            return qlh::stream_gemm_f16(static_cast<const uint16_t*>(xs.p), reinterpret_cast<const uint16_t*>(w),
+                                        static_cast<uint16_t*>(ys.p), M, N, K, stream) == hipSuccess;
         return hipblasLtMatmul(lt, plan.desc, &alpha, w, plan.a, xs.p, plan.b, &beta, ys.p, plan.c, ys.p,
-                               plan.c, &algo, wks.p, kWorkspace, stream) == HIPBLAS_STATUS_SUCCESS;
+                               plan.c, algo, wks.p, kWorkspace, stream) == HIPBLAS_STATUS_SUCCESS;
     };
     // time one candidate: kTuneReps launches over the weight copies, host wall clock
     // from the first launch to the stream's completion, so a candidate that launches
     // more kernels (e.g. a split-K reduction) pays their launch cost (-1: unsupported)
-    auto time_of = [&](const hipblasLtMatmulAlgo_t& algo, float& ms) -> hipError_t {
+    auto time_of = [&](const hipblasLtMatmulAlgo_t* algo, float& ms) -> hipError_t {
         ms = -1.0f;
         if (!run(algo, 0) || !run(algo, 1)) return hipSuccess;   // warm-up; unsupported: skip
         hipError_t r = hipStreamSynchronize(stream);
@@ -217,7 +232,7 @@ extern "C" hipError_t ql_gemm_tune_f16(int M, int N, int K, hipStream_t stream) 
     std::vector<std::pair<float, int>> first;
     for (int i = 0; i < (int)cands.size(); ++i) {
         float ms;
-        if ((e = time_of(cands[(size_t)i].algo, ms)) != hipSuccess) return e;
+        if ((e = time_of(&cands[(size_t)i].algo, ms)) != hipSuccess) return e;
         if (ms >= 0.0f) first.emplace_back(ms, i);
     }
     if (first.empty()) return hipErrorNotSupported;
@@ -227,13 +242,24 @@ extern "C" hipError_t ql_gemm_tune_f16(int M, int N, int K, hipStream_t stream) 
         if (first[i].second != 0) finalists.push_back(first[i].second);
     std::vector<double> total(finalists.size(), 0.0);
     std::vector<bool> valid(finalists.size(), true);
-    for (int round = 0; round < kTuneRounds; ++round)
+    // few rows: the weight-stream kernel, which ql_gemm_f16 runs there, against them
+    const bool stream_applies = qlh::stream_gemm_f16_applies(static_cast<const uint16_t*>(xs.p),
+                                                             static_cast<const uint16_t*>(ws_.p), M, N, K);
+    double stream_total = 0.0;
+    for (int round = 0; round < kTuneRounds; ++round) {
+        if (stream_applies) {
+            float ms;
+            if ((e = time_of(nullptr, ms)) != hipSuccess) return e;
+            if (ms < 0.0f) return hipErrorLaunchFailure;
+            stream_total += ms;
+        }
         for (size_t f = 0; f < finalists.size(); ++f) {
             float ms;
-            if ((e = time_of(cands[(size_t)finalists[f]].algo, ms)) != hipSuccess) return e;
+            if ((e = time_of(&cands[(size_t)finalists[f]].algo, ms)) != hipSuccess) return e;
             if (ms < 0.0f) valid[f] = false;
             total[f] += ms;
         }
+    }
     size_t pick = 0;
     for (size_t f = 1; f < finalists.size(); ++f)
         if (valid[f] && (!valid[pick] || total[f] < total[pick])) pick = f;
@@ -242,6 +268,8 @@ extern "C" hipError_t ql_gemm_tune_f16(int M, int N, int K, hipStream_t stream) 
     const hipblasLtMatmulAlgo_t best_algo = cands[(size_t)finalists[pick]].algo;
     if (best < 0.0f) return hipErrorNotSupported;
     std::lock_guard<std::mutex> lock(g_mu);
-    g_devices[dev].plans[std::make_tuple(M, N, K)].algo = best_algo;
+    Plan& chosen = g_devices[dev].plans[std::make_tuple(M, N, K)];
+    chosen.algo = best_algo;
+    chosen.over_stream = stream_applies && best * (1.0 + kTuneMargin) < stream_total;
     return hipSuccess;
 }
