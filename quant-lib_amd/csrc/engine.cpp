@@ -13,7 +13,7 @@
 //                                                     ql_attention_f16 on the QKV rows
 //                                                     for one fresh prompt
 //   x += a Wo^T; y = rmsnorm(x) * ffn_norm            hipBLASLt + ql_add_rmsnorm_f16
-//   delta_out = swiglu(y Wg^T, y Wu^T) Wd^T           hipBLASLt x2, ql_swiglu_f16, hipBLASLt
+//   delta_out = swiglu(y Wg^T, y Wu^T) Wd^T           hipBLASLt x2 (few rows: one launch), ql_swiglu_f16, hipBLASLt
 //
 // The MLP output is returned as delta_out and added by the next layer's fused
 // add+RMSNorm (or by ql_engine_logits_f16 after the last layer).  Weights are
@@ -25,6 +25,8 @@
 // allocated once at creation; the per-step calls allocate nothing (the GEMM
 // library context is created on the first fp16 GEMM).
 #include "quantlib_amd.h"
+#include "fp8_gemm_pair.hpp"
+#include "gemm_stream.hpp"
 
 #include <new>
 
@@ -60,6 +62,9 @@ struct GemmF16 {
         const uint16_t* m[] = {w->wqkv, w->wo, w->w_gate, w->w_up, w->w_down};
         return ql_gemm_f16(x, m[which], out, M, N, K, stream);
     }
+    hipError_t gate_up(const ql_engine* e, int M, int N, int K, hipStream_t stream) const {
+        return qlh::gemm_pair_f16(e->y, w->w_gate, e->g, w->w_up, e->u, M, N, K, stream);
+    }
 };
 
 struct GemmFp8 {
@@ -69,6 +74,11 @@ struct GemmFp8 {
         const ql_fp8_weight* m[] = {&w->wqkv, &w->wo, &w->w_gate, &w->w_up, &w->w_down};
         return ql_fp8_gemm_f16(x, m[which]->codes, m[which]->scales, M, N, K, w->format, w->granularity,
                                w->group_size, w->mode, out, e->fp8_ws, e->fp8_ws_bytes, stream);
+    }
+    hipError_t gate_up(const ql_engine* e, int M, int N, int K, hipStream_t stream) const {
+        return qlh::fp8_gemm_pair(e->y, w->w_gate.codes, w->w_gate.scales, e->g, w->w_up.codes, w->w_up.scales, e->u, M,
+                                  N, K, w->format, w->granularity, w->group_size, w->mode, e->fp8_ws, e->fp8_ws_bytes,
+                                  stream);
     }
 };
 
@@ -204,8 +214,7 @@ hipError_t layer_forward(ql_engine* e, const uint16_t* attn_norm, const uint16_t
     QL_TRY(gemm(e, e->attn, kWo, e->o, T, D, H * HD, stream));
     // MLP sublayer
     QL_TRY(ql_add_rmsnorm_f16(x, e->o, ffn_norm, e->y, T, D, d.rms_eps, stream));
-    QL_TRY(gemm(e, e->y, kWgate, e->g, T, F, D, stream));
-    QL_TRY(gemm(e, e->y, kWup, e->u, T, F, D, stream));
+    QL_TRY(gemm.gate_up(e, T, F, D, stream));
     QL_TRY(ql_swiglu_f16(e->g, e->u, e->mid, T, F, stream));
     QL_TRY(gemm(e, e->mid, kWdown, delta_out, T, D, F, stream));
     return hipSuccess;

@@ -34,6 +34,7 @@
 // slower, dequantizes into a workspace with the codec and runs the fp16 library GEMM.
 #include "ql_common.hpp"
 #include "fp8_decode.hpp"
+#include "fp8_gemm_pair.hpp"
 #include "fp8_gemm_tile.hpp"
 #include "stream_gemm.hpp"
 #include <type_traits>
@@ -737,6 +738,9 @@ struct SkinnyArgs {
     long long gs;         // group length in elements
     int groups_per_row;   // K / gs (kScaleGroup)
     int g_step, r_step;   // 256 / gs, 256 % gs: a wavefront's next chunk starts 256 k on
+    const char* W2;       // fp8_gemv, gridDim.y = 2: a second product of the same tokens and shape
+    const float* scales2;
+    _Float16* C2;
     int packed_a;         // register path: A holds the token fragments fragment-major
 };
 
@@ -1391,6 +1395,11 @@ template <int FMT, int MODE, int SK, int M>
 __global__ __launch_bounds__(kVecThreads) void fp8_gemv(SkinnyArgs p, int W, int J) {
     constexpr bool kScaled = !fold_scale<FMT, MODE, SK == kScaleGroupFold ? kScaleRow : SK>();
     extern __shared__ __align__(16) _Float16 tok[];   // [M][J * 1024]
+    if (blockIdx.y) {
+        p.W = p.W2;
+        p.scales = p.scales2;
+        p.C = p.C2;
+    }
     const int lane = threadIdx.x & (kWave - 1);
     const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * (kVecThreads / kWave) + threadIdx.x / kWave));
     const int KP = J * 1024;   // padded row length of the token tile
@@ -1712,7 +1721,7 @@ int gemv_kind(const Geom& g, int M, int K, int format, int mode, int& J) {
 template <int FMT, int MODE, int SK>
 void launch_gemv_sk(const SkinnyArgs& a, int J, hipStream_t st) {
     const int waves = std::min(a.N, kVecTargetWaves);
-    const dim3 grid((unsigned)((waves + kVecThreads / kWave - 1) / (kVecThreads / kWave))), block(kVecThreads);
+    const dim3 grid((unsigned)((waves + kVecThreads / kWave - 1) / (kVecThreads / kWave)), a.W2 ? 2 : 1), block(kVecThreads);
     const size_t lds = (size_t)a.M * (size_t)J * 1024u * sizeof(_Float16);
     if (a.M == 1) hipLaunchKernelGGL((fp8_gemv<FMT, MODE, SK, 1>), grid, block, lds, st, a, waves, J);
     else hipLaunchKernelGGL((fp8_gemv<FMT, MODE, SK, 2>), grid, block, lds, st, a, waves, J);
@@ -1793,7 +1802,7 @@ StreamPlan stream_plan(int M, int N, int K, size_t ws_bytes) {
 template <int FMT, int MODE, int SK, int MT>
 void launch_stream_mt(const StreamArgs& a, const StreamPlan& pl, hipStream_t st) {
     using WP = StreamFp8<FMT, MODE>;
-    const dim3 grid(qlh::blocks_for(a.N, 16 * pl.r), (unsigned)pl.splits), block(pl.nw * kWave);
+    const dim3 grid(qlh::blocks_for(a.N, 16 * pl.r), (unsigned)pl.splits, a.W2 ? 2 : 1), block(pl.nw * kWave);
     if (pl.r == 4) {
         if constexpr (MT < 4) hipLaunchKernelGGL((stream_gemm<WP, SK, MT, 4, 4>), grid, block, 0, st, a);
     } else if (pl.r == 2) {
@@ -2044,6 +2053,93 @@ extern "C" hipError_t ql_fp8_gemm_workspace_size(int M, int N, int K, int granul
     return hipSuccess;
 }
 
+namespace {
+
+// A second product of the same token rows by a matrix of the same shape and options.
+struct SecondWeights {
+    const uint8_t* W;
+    const float* scales;
+    uint16_t* C;
+};
+
+// The kernels that stream the weights once, for few token rows: launched where one
+// of them applies (and takes both products, if there are two), else false.
+bool few_rows(const uint16_t* A, const uint8_t* W, const float* scales, int M, int N, int K, const Geom& g, int format,
+              int mode, uint16_t* C, const SecondWeights* two, void* workspace, size_t workspace_bytes,
+              hipStream_t stream) {
+    if (!qlh::aligned16(A) || !qlh::aligned16(W) || (two && !qlh::aligned16(two->W))) return false;
+    int gemv_j = 0;
+    const int gkind = gemv_kind(g, M, K, format, mode, gemv_j);
+    if (gkind >= 0) {
+        SkinnyArgs a{};
+        a.A = reinterpret_cast<const char*>(A);
+        a.W = reinterpret_cast<const char*>(W);
+        a.scales = scales;
+        a.C = reinterpret_cast<_Float16*>(C);
+        if (two) {
+            a.W2 = reinterpret_cast<const char*>(two->W);
+            a.scales2 = two->scales;
+            a.C2 = reinterpret_cast<_Float16*>(two->C);
+        }
+        a.M = M;
+        a.N = N;
+        a.K = K;
+        a.gs = g.gs;
+        a.groups_per_row = K % g.gs == 0 ? (int)(K / g.gs) : 0;
+        QL_FP8_DISPATCH(format, mode, launch_gemv, a, gkind, gemv_j, stream);
+        return true;
+    }
+    if (!skinny_ok(M, N, K, g)) return false;
+    const bool ws_ok = workspace && qlh::aligned16(workspace) && ((uintptr_t)C & 7) == 0;
+    const int skind = stream_kind(g, M, N, K, format, mode);
+    const StreamPlan sp = skind >= 0 ? stream_plan(M, N, K, ws_ok ? workspace_bytes : 0) : StreamPlan{};
+    if (sp.r == 0 || (two && sp.splits > 1)) return false;
+    StreamArgs a{};
+    a.A = reinterpret_cast<const char*>(A);
+    a.W = reinterpret_cast<const char*>(W);
+    a.scales = scales;
+    a.C = reinterpret_cast<_Float16*>(C);
+    if (two) {
+        a.W2 = reinterpret_cast<const char*>(two->W);
+        a.scales2 = two->scales;
+        a.C2 = reinterpret_cast<_Float16*>(two->C);
+    }
+    a.M = M;
+    a.N = N;
+    a.K = K;
+    a.gs = (int)std::min<long long>(g.gs, K);
+    a.groups_per_row = g.n_groups == 1 ? 0 : K / a.gs;
+    a.part = static_cast<float*>(workspace);
+    a.chunks_per_split = sp.chunks_per_split;
+    QL_FP8_DISPATCH(format, mode, launch_stream, a, sp, skind, stream);
+    if (sp.splits > 1)
+        hipLaunchKernelGGL(splitk_reduce, dim3(qlh::blocks_for((long long)M * N / 4, kBlock)), dim3(kBlock), 0, stream,
+                           a.part, a.C, sp.splits, (long long)M * N);
+    return true;
+}
+
+}  // namespace
+
+// Gate and up of a decode step: two launches in a row fill and drain the chip twice; one
+// of both overlaps the second matrix with the first one's tail.  Two-layer steps on
+// MI355X, two launches -> one: one sequence over 2000 keys (4096 wide, FFN 14336, g128)
+// 213.2 -> 208.3 us, a drawn decode step 184.5 -> 174.8 us; bit-identical.  Not for
+// K-splits, whose partials would need a second area of the workspace.
+hipError_t qlh::fp8_gemm_pair(const uint16_t* A, const uint8_t* W, const float* scales, uint16_t* C, const uint8_t* W2,
+                              const float* scales2, uint16_t* C2, int M, int N, int K, int format, int granularity,
+                              int group_size, int mode, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+    Geom g;
+    const SecondWeights two{W2, scales2, C2};
+    if (decode_mode_ok(format, mode) && M > 0 && N > 0 && K > 0 && geom_for(N, K, granularity, group_size, g) && A && W &&
+        scales && C && W2 && scales2 && C2 &&
+        few_rows(A, W, scales, M, N, K, g, format, decode_mode(mode), C, &two, workspace, workspace_bytes, stream))
+        return hipGetLastError();
+    const hipError_t e = ql_fp8_gemm_f16(A, W, scales, M, N, K, format, granularity, group_size, mode, C, workspace,
+                                         workspace_bytes, stream);
+    return e != hipSuccess ? e : ql_fp8_gemm_f16(A, W2, scales2, M, N, K, format, granularity, group_size, mode, C2,
+                                                 workspace, workspace_bytes, stream);
+}
+
 extern "C" hipError_t ql_fp8_gemm_f16(const uint16_t* A, const uint8_t* W, const float* scales,
                                       int M, int N, int K, int format, int granularity,
                                       int group_size, int mode, uint16_t* C, void* workspace,
@@ -2054,46 +2150,11 @@ extern "C" hipError_t ql_fp8_gemm_f16(const uint16_t* A, const uint8_t* W, const
     if (M == 0 || N == 0) return hipSuccess;
     QL_CHECK_ARG(A && W && scales && C && K > 0);
     mode = decode_mode(mode);
-    int gemv_j = 0;
-    const int gkind = gemv_kind(g, M, K, format, mode, gemv_j);
-    if (gkind >= 0 && qlh::aligned16(A) && qlh::aligned16(W)) {
-        SkinnyArgs a{};
-        a.A = reinterpret_cast<const char*>(A);
-        a.W = reinterpret_cast<const char*>(W);
-        a.scales = scales;
-        a.C = reinterpret_cast<_Float16*>(C);
-        a.M = M;
-        a.N = N;
-        a.K = K;
-        a.gs = g.gs;
-        a.groups_per_row = K % g.gs == 0 ? (int)(K / g.gs) : 0;
-        QL_FP8_DISPATCH(format, mode, launch_gemv, a, gkind, gemv_j, stream);
+    if (few_rows(A, W, scales, M, N, K, g, format, mode, C, nullptr, workspace, workspace_bytes, stream))
         return hipGetLastError();
-    }
     if (skinny_ok(M, N, K, g) && qlh::aligned16(A) && qlh::aligned16(W)) {
         const bool ws_ok = workspace && qlh::aligned16(workspace) && ((uintptr_t)C & 7) == 0;
         const size_t ws = ws_ok ? workspace_bytes : 0;
-        const int skind = stream_kind(g, M, N, K, format, mode);
-        const StreamPlan sp = skind >= 0 ? stream_plan(M, N, K, ws) : StreamPlan{};
-        if (sp.r > 0) {
-            StreamArgs a{};
-            a.A = reinterpret_cast<const char*>(A);
-            a.W = reinterpret_cast<const char*>(W);
-            a.scales = scales;
-            a.C = reinterpret_cast<_Float16*>(C);
-            a.M = M;
-            a.N = N;
-            a.K = K;
-            a.gs = (int)std::min<long long>(g.gs, K);
-            a.groups_per_row = g.n_groups == 1 ? 0 : K / a.gs;
-            a.part = static_cast<float*>(workspace);
-            a.chunks_per_split = sp.chunks_per_split;
-            QL_FP8_DISPATCH(format, mode, launch_stream, a, sp, skind, stream);
-            if (sp.splits > 1)
-                hipLaunchKernelGGL(splitk_reduce, dim3(qlh::blocks_for((long long)M * N / 4, kBlock)), dim3(kBlock), 0,
-                                   stream, a.part, a.C, sp.splits, (long long)M * N);
-            return hipGetLastError();
-        }
         SkinnyPlan pl = skinny_plan(M, N, K, ws);
         // more than 32 tokens (four token tiles) on the register path: the token
         // rows are copied fragment-major after the split partials, when the

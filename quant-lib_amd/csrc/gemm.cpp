@@ -141,6 +141,16 @@ extern "C" hipError_t ql_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t
     return st == HIPBLAS_STATUS_SUCCESS ? hipSuccess : hipErrorLaunchFailure;
 }
 
+hipError_t qlh::gemm_pair_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, const uint16_t* w2, uint16_t* y2, int M,
+                              int N, int K, hipStream_t stream) {
+    int dev = 0;
+    if (x && w && y && w2 && y2 && M > 0 && N > 0 && K > 0 && stream_gemm_f16_applies(x, w, M, N, K) &&
+        stream_gemm_f16_applies(x, w2, M, N, K) && hipGetDevice(&dev) == hipSuccess && !tuned_to_library(dev, M, N, K))
+        return stream_gemm_f16(x, w, y, M, N, K, stream, w2, y2);
+    const hipError_t e = ql_gemm_f16(x, w, y, M, N, K, stream);
+    return e != hipSuccess ? e : ql_gemm_f16(x, w2, y2, M, N, K, stream);
+}
+
 namespace {
 
 // Scratch device memory of the tuner, released on every return path.

@@ -12,7 +12,7 @@ constexpr int kMaxTokens = 16;   // 17-32 tokens: the library is 0-6% faster on 
 
 template <int R>
 void launch(const StreamArgs& a, hipStream_t st) {
-    const dim3 grid(qlh::blocks_for(a.N, 16 * R)), block(8 * kWave);
+    const dim3 grid(qlh::blocks_for(a.N, 16 * R), 1, a.W2 ? 2 : 1), block(8 * kWave);
     hipLaunchKernelGGL((stream_gemm<StreamF16, kStreamNone, 1, R, 8>), grid, block, 0, st, a);
 }
 
@@ -35,11 +35,13 @@ bool qlh::stream_gemm_f16_applies(const uint16_t* x, const uint16_t* w, int M, i
 }
 
 hipError_t qlh::stream_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int N, int K,
-                                hipStream_t stream) {
+                                hipStream_t stream, const uint16_t* w2, uint16_t* y2) {
     StreamArgs a{};
     a.A = reinterpret_cast<const char*>(x);
     a.W = reinterpret_cast<const char*>(w);
     a.C = reinterpret_cast<_Float16*>(y);
+    a.W2 = reinterpret_cast<const char*>(w2);
+    a.C2 = reinterpret_cast<_Float16*>(y2);
     a.M = M;
     a.N = N;
     a.K = K;

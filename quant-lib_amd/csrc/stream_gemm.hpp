@@ -23,6 +23,9 @@ struct StreamArgs {
     int gs, groups_per_row;
     float* part;          // [splits][M][N] fp32 partials (gridDim.y > 1)
     int chunks_per_split; // K-split of blockIdx.y, in kStreamChunk steps
+    const char* W2;       // gridDim.z = 2: a second product of the same tokens and shape
+    const float* scales2; // (no K-split)
+    _Float16* C2;
 };
 
 constexpr int kStreamChunk = 128;       // k per step of a wavefront
@@ -58,6 +61,11 @@ __global__ __launch_bounds__(NW * kWave) void stream_gemm(StreamArgs p) {
     const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const int j = lane & 15, q = lane >> 4;
     const int n0 = blockIdx.x * 16 * R;
+    if (blockIdx.z) {
+        p.W = p.W2;
+        p.scales = p.scales2;
+        p.C = p.C2;
+    }
     const int rows = min(16 * R, p.N - n0);
     const uint32_t row_b = (uint32_t)p.K * WP::kBytes;
     // buffers that end at the workgroup's last weight row and the last token row:

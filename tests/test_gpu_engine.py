@@ -474,3 +474,21 @@ def test_argmax_any_alignment(cols, ld, f16):
     out = empty((rows,), np.int32)
     ql.call("ql_argmax_f16" if f16 else "ql_argmax_f32", d.ptr, rows, cols, ld, out.ptr, stream())
     assert list(host(out)) == list(want)
+
+
+# ---- gate and up in one launch ----------------------------------------------------------------
+# few-row steps take both matrices in one launch (1-2 rows, 3-64 rows, each scale kind); the
+# oracle's gate and up differ, so either one read or written in the other's place shows
+@pytest.mark.parametrize("fmt,gran,gs,mode", [
+    (ql.FP8_E4M3, ql.QUANT_PER_GROUP, 128, ql.FP8_MODE_REFERENCE),
+    (ql.FP8_E4M3, ql.QUANT_PER_GROUP, 64, ql.FP8_MODE_OCP),
+    (ql.FP8_E5M2, ql.QUANT_PER_CHANNEL, 0, ql.FP8_MODE_OCP),
+    (ql.FP8_E5M2, ql.QUANT_PER_GROUP, 128, ql.FP8_MODE_REFERENCE)])
+@pytest.mark.parametrize("prompts", [{0: 1}, {0: 3}, {0: 17, 1: 1}, {0: 49}])
+def test_engine_fp8_gate_and_up_of_few_rows(fmt, gran, gs, mode, prompts):
+    test_engine_fp8_layers_match_oracle(fmt, gran, gs, mode, prompts)
+
+
+@pytest.mark.parametrize("prompts", [{0: 1}, {0: 9, 1: 7}, {0: 9, 1: 8}])   # 16 rows take the stream, 17 do not
+def test_engine_f16_gate_and_up_of_few_rows(prompts):
+    test_engine_layers_steps_and_logits_match_oracle(prompts)
