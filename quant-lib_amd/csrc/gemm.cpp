@@ -30,7 +30,7 @@ struct Plan {
     hipblasLtMatmulDesc_t desc = nullptr;
     hipblasLtMatrixLayout_t a = nullptr, b = nullptr, c = nullptr;
     hipblasLtMatmulAlgo_t algo{};
-    bool over_stream = false;   // tuned, and faster than the weight-stream kernel
+    bool over_stream = false;   // tuned, and (where they were timed together) faster than the weight-stream kernel
 };
 
 struct Device {
@@ -88,7 +88,7 @@ hipError_t make_plan(Device& d, int M, int N, int K, Plan& p) {
     return hipSuccess;
 }
 
-// Whether ql_gemm_tune_f16 found the library faster than the weight-stream kernel.
+// Whether ql_gemm_tune_f16 chose the library for this shape.
 bool tuned_to_library(int dev, int M, int N, int K) {
     std::lock_guard<std::mutex> lock(g_mu);
     const auto d = g_devices.find(dev);
@@ -144,8 +144,8 @@ extern "C" hipError_t ql_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t
 hipError_t qlh::gemm_pair_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, const uint16_t* w2, uint16_t* y2, int M,
                               int N, int K, hipStream_t stream) {
     int dev = 0;
-    if (x && w && y && w2 && y2 && M > 0 && N > 0 && K > 0 && stream_gemm_f16_applies(x, w, M, N, K) &&
-        stream_gemm_f16_applies(x, w2, M, N, K) && hipGetDevice(&dev) == hipSuccess && !tuned_to_library(dev, M, N, K))
+    if (x && w && y && w2 && y2 && M > 0 && N > 0 && K > 0 && stream_gemm_f16_applies(x, w, M, N, K, true) &&
+        stream_gemm_f16_applies(x, w2, M, N, K, true) && hipGetDevice(&dev) == hipSuccess && !tuned_to_library(dev, M, N, K))
         return stream_gemm_f16(x, w, y, M, N, K, stream, w2, y2);
     const hipError_t e = ql_gemm_f16(x, w, y, M, N, K, stream);
     return e != hipSuccess ? e : ql_gemm_f16(x, w2, y2, M, N, K, stream);
@@ -280,6 +280,6 @@ extern "C" hipError_t ql_gemm_tune_f16(int M, int N, int K, hipStream_t stream) 
     std::lock_guard<std::mutex> lock(g_mu);
     Plan& chosen = g_devices[dev].plans[std::make_tuple(M, N, K)];
     chosen.algo = best_algo;
-    chosen.over_stream = stream_applies && best * (1.0 + kTuneMargin) < stream_total;
+    chosen.over_stream = !stream_applies || best * (1.0 + kTuneMargin) < stream_total;
     return hipSuccess;
 }

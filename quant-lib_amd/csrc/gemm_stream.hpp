@@ -7,8 +7,9 @@
 
 namespace qlh {
 
-// Whether the weight-stream kernel takes y[M, N] = x[M, K] w[N, K]^T.
-bool stream_gemm_f16_applies(const uint16_t* x, const uint16_t* w, int M, int N, int K);
+// Whether the weight-stream kernel takes y[M, N] = x[M, K] w[N, K]^T (pair: together
+// with a second matrix).
+bool stream_gemm_f16_applies(const uint16_t* x, const uint16_t* w, int M, int N, int K, bool pair = false);
 // w2: a second matrix of the same shape, y2 = x w2^T in the same launch.
 hipError_t stream_gemm_f16(const uint16_t* x, const uint16_t* w, uint16_t* y, int M, int N, int K, hipStream_t stream,
                            const uint16_t* w2 = nullptr, uint16_t* y2 = nullptr);

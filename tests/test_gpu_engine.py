@@ -12,6 +12,7 @@ every stage to binary16 (2^-11 relative) but accumulate GEMMs in different
 orders (fp32 in hipBLASLt, double in the oracle), so single-ulp differences in
 intermediate values propagate through up to six dependent stages."""
 import ctypes
+import sys
 
 import numpy as np
 import pytest
@@ -491,4 +492,11 @@ def test_engine_fp8_gate_and_up_of_few_rows(fmt, gran, gs, mode, prompts):
 
 @pytest.mark.parametrize("prompts", [{0: 1}, {0: 9, 1: 7}, {0: 9, 1: 8}])   # 16 rows take the stream, 17 do not
 def test_engine_f16_gate_and_up_of_few_rows(prompts):
+    test_engine_layers_steps_and_logits_match_oracle(prompts)
+
+
+# more than 8192 FFN rows: 17-32 token rows too (the last 64-row tile is 8 rows), 33 not
+@pytest.mark.parametrize("prompts", [{0: 9, 1: 8}, {0: 30, 1: 2}, {0: 33}])
+def test_engine_f16_gate_and_up_of_a_large_ffn(prompts, monkeypatch):
+    monkeypatch.setattr(sys.modules[__name__], "FF", 8264)
     test_engine_layers_steps_and_logits_match_oracle(prompts)
