@@ -8,7 +8,8 @@ namespace {
 
 using namespace ql;
 
-constexpr int kMaxTokens = 16;   // 17-32 tokens: the library is 0-6% faster on most shapes
+constexpr int kMaxTokens = 16;   // 17-32 tokens: the library is 0-6% faster on most shapes,
+constexpr int kManyRows = 16384; // but not on more weight rows than this in a launch
 
 template <int R, int MT = 1, int NW = 8>
 void launch(const StreamArgs& a, hipStream_t st) {
@@ -31,9 +32,10 @@ void launch(const StreamArgs& a, hipStream_t st) {
 // 13.0 / 13.5 / 18.0).
 // Two products of the same rows (gate and up) in one launch save one fill and drain of
 // the chip, which turns 17-32 rows of large matrices in the kernel's favour: a decode
-// step of 32 sequences, two layers of 4096 with FFN 14336 and logits, 398 -> 387 us.
+// step of 32 sequences, two layers of 4096 with FFN 14336 and logits, 398 -> 387 us (both in 44.9 us, 5.2 TB/s;
+// the library on the 32000 x 4096 logits 59.2 us, 4.4 TB/s, which come here too).
 bool qlh::stream_gemm_f16_applies(const uint16_t* x, const uint16_t* w, int M, int N, int K, bool pair) {
-    if (M > (pair && N > 8192 ? 2 : 1) * kMaxTokens || K % kStreamChunk || K > kStreamMaxK || !qlh::aligned16(x) || !qlh::aligned16(w)) return false;
+    if (M > ((pair ? 2 : 1) * (long long)N > kManyRows ? 2 : 1) * kMaxTokens || K % kStreamChunk || K > kStreamMaxK || !qlh::aligned16(x) || !qlh::aligned16(w)) return false;
     return N > 4096 ? K <= 4096 : K <= 8192 || N >= 3072;
 }
 

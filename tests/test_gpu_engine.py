@@ -500,3 +500,19 @@ def test_engine_f16_gate_and_up_of_few_rows(prompts):
 def test_engine_f16_gate_and_up_of_a_large_ffn(prompts, monkeypatch):
     monkeypatch.setattr(sys.modules[__name__], "FF", 8264)
     test_engine_layers_steps_and_logits_match_oracle(prompts)
+
+
+# 17-32 rows of one matrix past 16384 weight rows (16392: the last 64-row tile is 8 rows)
+@pytest.mark.parametrize("M,N,K", [(17, 16392, 128), (32, 16392, 384), (33, 16392, 128), (17, 16384, 128)])
+def test_gemm_f16_of_many_weight_rows(M, N, K):
+    x = to_f16_bits(normal(91 + M, (M, K)))
+    w = to_f16_bits(normal(92 + K, (N, K)) * np.float32(K ** -0.5))
+    want = f16_bits_to_f32(orc.matmul(x, w)).astype(np.float64)
+    y = empty((M * N,), np.uint16)
+    dx, dw = dev(x), dev(w)
+    ql.call("ql_gemm_f16", dx.ptr, dw.ptr, y.ptr, M, N, K, stream())
+    got = f16_bits_to_f32(host(y, shape=(M, N))).astype(np.float64)
+    # fp32 accumulation in any order, one binary16 rounding of the result
+    bound = 2.0 ** -10 * np.abs(want) + 2.0 ** -10 * (
+        np.abs(f16_bits_to_f32(x)).astype(np.float64) @ np.abs(f16_bits_to_f32(w)).T.astype(np.float64))
+    assert np.all(np.abs(got - want) <= bound)
